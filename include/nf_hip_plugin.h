@@ -111,7 +111,7 @@ NF_API nf_status nf_hip_plan_dispatch(const char *op_name,
 
 /* Batch-size switch points between the kernel families of the fused ops:
  * the VALU decode GEMV while M <= gemv_max_m, the small-batch MFMA kernel
- * above it up to skinny_max_m (at most 32 f32 / 64 f16 activation rows per
+ * above it up to skinny_max_m (at most 64 f32 / 128 f16 activation rows per
  * launch), the tiled MFMA GEMM beyond (f16 activations: fp16 MFMA; f32
  * activations: exact bf16 pieces on bf16 MFMA, K % 64 == 0).  f16 and f32
  * activations each have their own switch points.  Defaults come from

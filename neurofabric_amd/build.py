@@ -35,6 +35,7 @@ HIP_SOURCES = [
     CSRC / "kernels" / "gemv.hip",
     CSRC / "kernels" / "gemm.hip",
     CSRC / "kernels" / "skinny.hip",
+    CSRC / "kernels" / "skinny_ring.hip",
     CSRC / "kernels" / "generic.hip",
     CSRC / "kernels" / "dense.hip",
     CSRC / "kernels" / "layer.hip",

@@ -50,13 +50,17 @@ hipError_t launch_gemv_group(QFmt q, EType t, const void* A, const GemvJob* jobs
 hipError_t launch_skinny_group(QFmt q, EType t, const void* A, const GemvJob* jobs, uint32_t n, uint32_t M,
                                uint32_t K, const Workspace& ws, hipStream_t s);
 
-// Small-batch (M <= 64) MFMA kernel; skinny_fits() says whether a shape and
-// operand alignment suit it.
+// Small-batch MFMA kernels (f32 up to 64 rows a launch, f16 up to 128);
+// skinny_fits() says whether a shape and operand alignment suit them,
+// ring_serves() which shapes launch_skinny hands to the ring kernel.
+bool ring_serves(QFmt q, EType t, uint32_t M, uint32_t N, uint32_t K);
+hipError_t launch_skinny_ring(QFmt q, const void* A, const GemvJob* jobs, uint32_t n, uint32_t M, uint32_t K,
+                              const Workspace& ws, hipStream_t s);
 bool skinny_fits(uint32_t M, uint32_t N, uint32_t K, const void* A, const void* W);
 uint32_t skinny_max_rows(EType t);  // activation rows per launch
 hipError_t launch_skinny(QFmt q, EType t, const void* A, const void* W, void* C, uint32_t M, uint32_t N,
                          uint32_t K, const Workspace& ws, hipStream_t s);
-// Several small-batch linears over the same activations (M <= 32, same
+// Several small-batch linears over the same activations (same
 // format, dtype and K) in one launch, each computed exactly as launch_skinny
 // would; hipErrorNotSupported when they would not get the same kernel
 // variant and K split on their own (the caller launches them one by one).

@@ -73,8 +73,8 @@ struct LayerParams {
 // Switch points between the kernel families of the fused op: the VALU GEMV
 // while M <= gemv_max_m (and its activation stage fits in LDS), the
 // small-batch MFMA kernel while M <= skinny_max_m (f16 and f32 activations
-// each have their own; the f32 ring kernel takes all 64 rows in one launch),
-// the tiled MFMA GEMM above (f16: fp16 MFMA; f32: bf16-piece MFMA, K % 64 == 0, else the GEMV).
+// each have their own), the tiled MFMA GEMM above (f16: fp16 MFMA, whose
+// launcher leaves batches up to 64 or 128 rows to the small-batch kernel; f32: bf16-piece MFMA, K % 64 == 0, else the GEMV).
 // Defaults from measured sweeps on MI355X (graph replay over 4 rotated weight
 // copies).  bench.py's configs[4] section (28672x8192 and 8192x28672 Q4_0,
 // f16 activations): the GEMV is fastest up to M = 2 (31.0 / 38.8 us against
@@ -97,7 +97,7 @@ struct LayerParams {
 // only while the weights are at most gemv_m4_max_weight_bytes (16 MB).
 // skinny_f16_max_k caps K for f16 batches above M = 4 on the small-batch
 // kernel (longer K goes to the tiled GEMM); no cap by default, since the
-// small-batch kernel's K split over workgroups (skinny_split) makes it the
+// small-batch kernel's K split over workgroups makes it the
 // faster one at K = 28672 too (M = 8: 52.8 against 68.1 us).
 struct Tuning {
   uint32_t gemv_max_m_f32 = 4;

@@ -725,14 +725,18 @@ nf_status launch(Provider* p, const Prepared* prs, uint32_t n) {
       GemvJob jobs[kGemvGroupMax];
       for (uint32_t j = 0; j < n; ++j) jobs[j] = GemvJob{prs[j].in[1]->dev, prs[j].out[0]->dev, prs[j].pl.N};
       const Plan& pl = prs[0].pl;
-      e = pl.path == Path::Gemv ? launch_gemv_group(pl.q, pl.c, prs[0].in[0]->dev, jobs, n, pl.M, pl.K, p->stream)
-                                : launch_skinny_group(pl.q, pl.c, prs[0].in[0]->dev, jobs, n, pl.M, pl.K, p->ws,
-                                                      p->stream);
-      if (e == hipErrorNotSupported) {
-        p->launch_groups.fetch_add(n - 1, std::memory_order_relaxed);
-        e = hipSuccess;
-        for (uint32_t j = 0; j < n && e == hipSuccess; ++j)
-          e = run_plan(prs[j].pl, prs[j].in, prs[j].out, p->tuning.gemm_tile, p->ws, p->stream);
+      // One launch for the group; if the kernel declines, the first job on
+      // its own and then the rest the same way.
+      for (uint32_t j0 = 0; j0 < n && e == hipSuccess;) {
+        e = hipErrorNotSupported;
+        if (n - j0 > 1)
+          e = pl.path == Path::Gemv
+                  ? launch_gemv_group(pl.q, pl.c, prs[0].in[0]->dev, jobs + j0, n - j0, pl.M, pl.K, p->stream)
+                  : launch_skinny_group(pl.q, pl.c, prs[0].in[0]->dev, jobs + j0, n - j0, pl.M, pl.K, p->ws, p->stream);
+        if (e != hipErrorNotSupported) break;
+        if (n - j0 > 1) p->launch_groups.fetch_add(1, std::memory_order_relaxed);
+        e = run_plan(prs[j0].pl, prs[j0].in, prs[j0].out, p->tuning.gemm_tile, p->ws, p->stream);
+        ++j0;
       }
     }
     if (rec) (void)hipEventRecord(rec->stop, p->stream);

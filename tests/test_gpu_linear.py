@@ -171,6 +171,34 @@ def test_skinny_ring_f32_edges(provider, oracle_mod, fmt, shape):
 
 @pytest.mark.parametrize("fmt", ["q4_0", "q8_0"])
 @pytest.mark.parametrize("f16", [False, True], ids=["f32", "f16"])
+@pytest.mark.parametrize("shape", [(1, 1, 256), (7, 33, 1280), (16, 15, 768), (33, 513, 5376), (64, 129, 2304),
+                                   (65, 150, 768), (128, 257, 1792)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_skinny_partial_chunks(provider, oracle_mod, fmt, f16, shape):
+    """Small-batch kernel where K is no multiple of its chunk (512 for f16
+    Q4_0, 256 or 128 else): the last chunk's loads past the row's end must
+    read zeros, not the next row.  One row and one column, ragged tiles, and
+    every count of 16-row activation tiles; twice in a row (split-K
+    counters).  The next row's blocks hold infinite scales in every second
+    row, so a byte of them in a finite row's sum shows."""
+    M, N, K = shape
+    old = provider.get_tuning()
+    W = syn.weights(fmt, N, K, seed=M + N).reshape(N, K // 32, -1).copy()
+    W[1::2, :, 0], W[1::2, :, 1] = 0x00, 0x7C  # fp16 +inf scales
+    A = syn.activations(M, K, seed=K, dtype=np.float16 if f16 else np.float32)
+    ref = oracle_mod.fused(A, W.reshape(-1), fmt, M, N, K, f16=f16, threads=8)
+    ref = (ref.view(np.float16) if f16 else ref).reshape(M, N)[:, ::2].astype(np.float32)
+    try:
+        _force_path(provider, "skinny", f16)
+        for rep in range(2):
+            got = run_fused(provider, fmt, A, W.reshape(-1), M, N, K, f16).astype(np.float32)
+            assert_close(got[:, ::2], ref, what=f"{fmt} f16={f16} {M}x{N}x{K} call {rep}")
+    finally:
+        provider.set_tuning(old)
+
+
+@pytest.mark.parametrize("fmt", ["q4_0", "q8_0"])
+@pytest.mark.parametrize("f16", [False, True], ids=["f32", "f16"])
 @pytest.mark.parametrize("shape", [(4, 300, 4096), (3, 130, 5632), (4, 64, 7168)], ids=lambda s: "x".join(map(str, s)))
 def test_gemv_large_activation_staging(provider, oracle_mod, fmt, f16, shape):
     """GEMV with the activations' LDS stage above 64 KB (opt-in dynamic LDS):
