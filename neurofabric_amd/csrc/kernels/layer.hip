@@ -10,6 +10,8 @@
 // accurate expf / tanhf / powf / sincosf / sqrt; row reductions (rms_norm's
 // sum of squares, softmax's sum) are tree sums in fp32 rather than the
 // reference's sequential loop, so those ops agree with it to rounding.
+#include <type_traits>
+
 #include "../launch.hpp"
 #include "common.hpp"
 
@@ -69,6 +71,32 @@ __global__ __launch_bounds__(kThreads) void unary_kernel(const T* __restrict__ i
   }
 }
 
+// silu and the elementwise_mul of its output with `up`, both outputs written
+// (act may be gate or out; each element is read and written by one thread).
+// Bound by the launch at decode sizes, by HBM above: the second kernel's read
+// of act is saved.  5632 f32 elements: 2.4 + 2.3 us as two launches -> 2.5.
+template <typename T>
+__global__ __launch_bounds__(kThreads) void silu_mul_kernel(const T* gate, const T* up, T* act, T* out, uint64_t n) {
+  constexpr int V = 16 / (int)sizeof(T);
+  typedef T vec_t __attribute__((ext_vector_type(V)));
+  const uint64_t i0 = ((uint64_t)blockIdx.x * kThreads + threadIdx.x) * V;
+  if (i0 >= n) return;
+  if (i0 + V <= n) {
+    vec_t x = *reinterpret_cast<const vec_t*>(gate + i0);
+    const vec_t y = *reinterpret_cast<const vec_t*>(up + i0);
+#pragma unroll
+    for (int j = 0; j < V; ++j) x[j] = (T)unary_f<EwFnK::Silu>((float)x[j]);
+    *reinterpret_cast<vec_t*>(act + i0) = x;
+    *reinterpret_cast<vec_t*>(out + i0) = x * y;
+  } else {
+    for (uint64_t i = i0; i < n; ++i) {
+      const T y = up[i], x = (T)unary_f<EwFnK::Silu>((float)gate[i]);
+      act[i] = x;
+      out[i] = (T)(x * y);
+    }
+  }
+}
+
 // attention_prefill mock: k = x * 0.5, v = x * -0.25 (metal_provider.mm:56-66).
 __global__ __launch_bounds__(kThreads) void mock_prefill_kernel(const float* __restrict__ in, float* __restrict__ k,
                                                                 float* __restrict__ v, uint64_t nk, uint64_t nv) {
@@ -120,21 +148,30 @@ __global__ __launch_bounds__(kThreads) void rms_norm_kernel(const T* __restrict_
 }
 
 // The same with the row held in registers: 16-byte loads (NC per thread,
-// all issued before the sum; a chunk past the row re-reads the row's last
-// chunk and counts 0), then 16-byte stores.  dim % (16 / sizeof(T)) == 0.
-template <typename T, int NC>
-__global__ __launch_bounds__(kThreads) void rms_norm_vec_kernel(const T* __restrict__ in,
+// all issued before the sum, the weights' too, so the row costs one memory
+// round trip; a chunk past the row re-reads the row's last chunk and counts
+// 0), then 16-byte stores.  dim % (16 / sizeof(T)) == 0.
+// ADD: the row is in + in2, stored to `sum` as well (the residual addition
+// before the norm; `sum` may be in or in2).  One launch for the two, and the
+// norm's read of the sum saved: 2048 f32, 2.3 + 3.3 us -> 2.9.
+template <typename T, int NC, bool ADD>
+__global__ __launch_bounds__(kThreads) void rms_norm_vec_kernel(const T* in, const T* in2, T* sum,
                                                                 const float* __restrict__ w,
                                                                 T* __restrict__ out, uint32_t dim, float eps) {
   constexpr int VW = 16 / sizeof(T);
   typedef T VecT __attribute__((ext_vector_type(VW)));
+  typedef float F4 __attribute__((ext_vector_type(4), aligned(4)));  // the weights may have any float alignment
   __shared__ float red[4];
   const uint64_t base = (uint64_t)blockIdx.x * dim;
   VecT v[NC];
+  F4 wv[NC][VW / 4];
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
-    const uint32_t j = (c * kThreads + threadIdx.x) * VW;
-    v[c] = *reinterpret_cast<const VecT*>(in + base + (j < dim ? j : dim - VW));
+    const uint32_t j = (c * kThreads + threadIdx.x) * VW, jj = j < dim ? j : dim - VW;
+    v[c] = *reinterpret_cast<const VecT*>(in + base + jj);
+    if constexpr (ADD) v[c] += *reinterpret_cast<const VecT*>(in2 + base + jj);
+#pragma unroll
+    for (int e = 0; e < VW / 4; ++e) wv[c][e] = *reinterpret_cast<const F4*>(w + jj + 4 * e);
   }
   float ss = 0.0f;
 #pragma unroll
@@ -151,9 +188,10 @@ __global__ __launch_bounds__(kThreads) void rms_norm_vec_kernel(const T* __restr
   for (int c = 0; c < NC; ++c) {
     const uint32_t j = (c * kThreads + threadIdx.x) * VW;
     if (j >= dim) continue;
+    if constexpr (ADD) *reinterpret_cast<VecT*>(sum + base + j) = v[c];
     VecT o;
 #pragma unroll
-    for (int e = 0; e < VW; ++e) o[e] = (T)((float)v[c][e] * rms * w[j + e]);
+    for (int e = 0; e < VW; ++e) o[e] = (T)((float)v[c][e] * rms * wv[c][e / 4][e % 4]);
     *reinterpret_cast<VecT*>(out + base + j) = o;
   }
 }
@@ -352,33 +390,45 @@ __global__ __launch_bounds__(64) void argmax_merge_kernel(const float* __restric
 // One thread per (group of rows at one position, pair p): the rotation of
 // pair p is computed once and applied to every row of the group (up to
 // kRopeRows of the n_heads rows of a token for rope_batch, a divisor of
-// n_heads so no group spans two tokens; kRopeRows rows for rope).  Small
-// groups keep many threads in flight: each row is a dependent load / store.
+// n_heads so no group spans two tokens; kRopeRows rows for rope).  A launch
+// of few rows is bound by a thread's chain of dependent loads and stores, so
+// groups shrink until the launch has 256 workgroups: 32 heads of 64 at one
+// position, 4.1 us with groups of 8, 2.6 with groups of 1.
+// A launch takes one job, or two of the same head_dim, step and theta (a
+// layer's q and k), the second's workgroups after the first's.
 constexpr uint32_t kRopeRows = 8;
 
 template <typename T>
-__global__ __launch_bounds__(kThreads) void rope_kernel(const T* __restrict__ in, T* __restrict__ out, uint64_t rows,
-                                                        uint32_t head_dim, uint32_t rows_per_group,
-                                                        uint32_t rows_per_pos, uint32_t step, float theta,
-                                                        bool batch) {
+struct RopeJob {
+  const T* in;
+  T* out;
+  uint64_t rows;
+  uint32_t rows_per_group, rows_per_pos;
+};
+
+template <typename T>
+__global__ __launch_bounds__(kThreads) void rope_kernel(RopeJob<T> j0, RopeJob<T> j1, uint32_t wgs0,
+                                                        uint32_t head_dim, uint32_t step, float theta, bool batch) {
+  const bool second = blockIdx.x >= wgs0;
+  const RopeJob<T> job = second ? j1 : j0;
   const uint32_t half = head_dim / 2;
-  const uint64_t id = (uint64_t)blockIdx.x * kThreads + threadIdx.x;
+  const uint64_t id = (uint64_t)(blockIdx.x - (second ? wgs0 : 0)) * kThreads + threadIdx.x;
   const uint64_t grp = id / half;
   const uint32_t pair = (uint32_t)(id % half);
-  const uint64_t r0 = grp * rows_per_group;
-  if (r0 >= rows) return;
-  const uint64_t pos = batch ? r0 / rows_per_pos + step : step;
+  const uint64_t r0 = grp * job.rows_per_group;
+  if (r0 >= job.rows) return;
+  const uint64_t pos = batch ? r0 / job.rows_per_pos + step : step;
   const float freq = 1.0f / powf(theta, (float)(2 * pair) / (float)head_dim);
   const float angle = (float)pos * freq;
   float s, c;
   sincosf(angle, &s, &c);
-  const uint64_t r1 = min(rows, r0 + rows_per_group);
+  const uint64_t r1 = min(job.rows, r0 + job.rows_per_group);
   for (uint64_t r = r0; r < r1; ++r) {
     const uint64_t base = r * head_dim;
-    const float x0 = (float)in[base + pair];
-    const float x1 = (float)in[base + pair + half];
-    out[base + pair] = (T)(x0 * c - x1 * s);
-    out[base + pair + half] = (T)(x0 * s + x1 * c);
+    const float x0 = (float)job.in[base + pair];
+    const float x1 = (float)job.in[base + pair + half];
+    job.out[base + pair] = (T)(x0 * c - x1 * s);
+    job.out[base + pair + half] = (T)(x0 * s + x1 * c);
   }
 }
 
@@ -554,29 +604,39 @@ hipError_t launch_mock_prefill(const void* in, void* k, void* v, uint64_t nk, ui
   return hipGetLastError();
 }
 
+// 16-byte chunks of a row per thread, rounded up to 1, 2, 4 or 8; 0 where
+// rms_norm_vec_kernel does not take the row.
+static int rms_chunks(EType t, const void* in, const void* out, uint32_t dim) {
+  // rows held in registers when they split into 16-byte chunks, at most 8
+  // per thread (8192 f16 / 4096 f32 elements per 4 chunks, twice that for 8)
+  const uint32_t vw = t == EType::F16 ? 8u : 4u, per = nfk::layer::kThreads * vw;
+  const uint32_t chunks = (dim + per - 1) / per;
+  if (!nfk::layer::a16(in) || !nfk::layer::a16(out) || dim % vw != 0 || dim < vw || chunks > 8) return 0;
+  return chunks <= 1 ? 1 : chunks <= 2 ? 2 : chunks <= 4 ? 4 : 8;
+}
+
+template <typename T, bool ADD>
+static hipError_t rms_vec(int nc, const void* in, const void* in2, void* sum, const void* w, void* out, uint32_t rows,
+                          uint32_t dim, float eps, hipStream_t s) {
+  using namespace nfk::layer;
+  auto go = [&](auto c) {
+    rms_norm_vec_kernel<T, decltype(c)::value, ADD><<<rows, kThreads, 0, s>>>(
+        (const T*)in, (const T*)in2, (T*)sum, (const float*)w, (T*)out, dim, eps);
+  };
+  if (nc == 1) go(std::integral_constant<int, 1>{});
+  else if (nc == 2) go(std::integral_constant<int, 2>{});
+  else if (nc == 4) go(std::integral_constant<int, 4>{});
+  else go(std::integral_constant<int, 8>{});
+  return hipGetLastError();
+}
+
 hipError_t launch_rms_norm(EType t, const void* in, const void* w, void* out, uint32_t rows, uint32_t dim, float eps,
                            hipStream_t s) {
   if (rows == 0) return hipSuccess;
   using namespace nfk::layer;
-  // rows held in registers when they split into 16-byte chunks, at most 8
-  // per thread (8192 f16 / 4096 f32 elements per 4 chunks, twice that for 8)
-  const uint32_t vw = t == EType::F16 ? 8u : 4u;
-  const bool aligned = ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) % 16) == 0;
-  const uint32_t chunks = (dim + kThreads * vw - 1) / (kThreads * vw);
-  if (aligned && dim % vw == 0 && dim >= vw && chunks <= 8) {
-    const int nc = chunks <= 1 ? 1 : chunks <= 2 ? 2 : chunks <= 4 ? 4 : 8;
-#define NF_RMS_VEC(TT, NC)                                                                                      \
-  rms_norm_vec_kernel<TT, NC><<<rows, kThreads, 0, s>>>((const TT*)in, (const float*)w, (TT*)out, dim, eps)
-    if (t == EType::F16) {
-      if (nc == 1) NF_RMS_VEC(half_t, 1); else if (nc == 2) NF_RMS_VEC(half_t, 2);
-      else if (nc == 4) NF_RMS_VEC(half_t, 4); else NF_RMS_VEC(half_t, 8);
-    } else {
-      if (nc == 1) NF_RMS_VEC(float, 1); else if (nc == 2) NF_RMS_VEC(float, 2);
-      else if (nc == 4) NF_RMS_VEC(float, 4); else NF_RMS_VEC(float, 8);
-    }
-#undef NF_RMS_VEC
-    return hipGetLastError();
-  }
+  if (const int nc = rms_chunks(t, in, out, dim))
+    return t == EType::F16 ? rms_vec<half_t, false>(nc, in, nullptr, nullptr, w, out, rows, dim, eps, s)
+                           : rms_vec<float, false>(nc, in, nullptr, nullptr, w, out, rows, dim, eps, s);
   if (t == EType::F16)
     rms_norm_kernel<half_t><<<rows, kThreads, 0, s>>>((const half_t*)in, (const float*)w, (half_t*)out, dim, eps);
   else
@@ -584,26 +644,54 @@ hipError_t launch_rms_norm(EType t, const void* in, const void* w, void* out, ui
   return hipGetLastError();
 }
 
-hipError_t launch_rope(EType t, bool batch, const void* in, void* out, uint64_t n, uint32_t n_heads,
-                       uint32_t head_dim, uint32_t step, float theta, hipStream_t s) {
-  if (n == 0) return hipSuccess;
+hipError_t launch_add_rms_norm(EType t, const void* a, const void* b, void* sum, const void* w, void* out,
+                               uint32_t rows, uint32_t dim, float eps, hipStream_t s) {
   using namespace nfk::layer;
-  const uint64_t rows = n / head_dim;
-  if (batch && n_heads == 0) return hipErrorInvalidValue;  // the planner rejects it first
-  uint32_t per = kRopeRows;  // rows sharing one position and one rotation
-  if (batch) {
-    per = n_heads < kRopeRows ? n_heads : kRopeRows;
-    while (n_heads % per) --per;
-  }
-  const uint64_t groups = (rows + per - 1) / per;
-  const uint64_t threads = groups * (head_dim / 2);
+  const int nc = a16(a) && a16(b) ? rms_chunks(t, sum, out, dim) : 0;
+  if (nc == 0 || rows == 0) return hipErrorNotSupported;
+  return t == EType::F16 ? rms_vec<half_t, true>(nc, a, b, sum, w, out, rows, dim, eps, s)
+                         : rms_vec<float, true>(nc, a, b, sum, w, out, rows, dim, eps, s);
+}
+
+hipError_t launch_silu_mul(EType t, const void* gate, const void* up, void* act, void* out, uint64_t n, hipStream_t s) {
+  using namespace nfk::layer;
+  if (n == 0 || !a16(gate) || !a16(up) || !a16(act) || !a16(out)) return hipErrorNotSupported;
   if (t == EType::F16)
-    rope_kernel<half_t><<<grid_for(threads), kThreads, 0, s>>>((const half_t*)in, (half_t*)out, rows, head_dim, per,
-                                                               n_heads, step, theta, batch);
+    silu_mul_kernel<half_t><<<grid_for((n + 7) / 8), kThreads, 0, s>>>((const half_t*)gate, (const half_t*)up,
+                                                                       (half_t*)act, (half_t*)out, n);
   else
-    rope_kernel<float><<<grid_for(threads), kThreads, 0, s>>>((const float*)in, (float*)out, rows, head_dim, per,
-                                                              n_heads, step, theta, batch);
+    silu_mul_kernel<float><<<grid_for((n + 3) / 4), kThreads, 0, s>>>((const float*)gate, (const float*)up,
+                                                                      (float*)act, (float*)out, n);
   return hipGetLastError();
+}
+
+template <typename T>
+static hipError_t rope_jobs(bool batch, const RopeArgs* args, uint32_t njobs, uint32_t head_dim, uint32_t step,
+                            float theta, hipStream_t s) {
+  using namespace nfk::layer;
+  RopeJob<T> jobs[2] = {};
+  uint64_t wgs[2] = {0, 0};
+  for (uint32_t i = 0; i < njobs; ++i) {
+    const RopeArgs& a = args[i];
+    if (batch && a.n_heads == 0) return hipErrorInvalidValue;  // the planner rejects it first
+    const uint64_t rows = a.n / head_dim;
+    uint32_t per = batch && a.n_heads < kRopeRows ? a.n_heads : kRopeRows;  // rows sharing one position and one rotation
+    while (per > 1 && ((batch && a.n_heads % per != 0) ||
+                       (rows + per - 1) / per * (head_dim / 2) < 256ull * kThreads))
+      --per;
+    jobs[i] = RopeJob<T>{(const T*)a.in, (T*)a.out, rows, per, a.n_heads};
+    wgs[i] = ((rows + per - 1) / per * (head_dim / 2) + kThreads - 1) / kThreads;
+  }
+  if (wgs[0] + wgs[1] == 0) return hipSuccess;
+  rope_kernel<T><<<dim3((unsigned)(wgs[0] + wgs[1])), kThreads, 0, s>>>(jobs[0], jobs[1], (uint32_t)wgs[0], head_dim,
+                                                                       step, theta, batch);
+  return hipGetLastError();
+}
+
+hipError_t launch_rope(EType t, bool batch, const RopeArgs* jobs, uint32_t n_jobs, uint32_t head_dim, uint32_t step,
+                       float theta, hipStream_t s) {
+  return t == EType::F16 ? rope_jobs<nfk::half_t>(batch, jobs, n_jobs, head_dim, step, theta, s)
+                         : rope_jobs<float>(batch, jobs, n_jobs, head_dim, step, theta, s);
 }
 
 // Rows wider than two chunks, with room for their partials in the

@@ -94,9 +94,23 @@ hipError_t launch_unary(EwFn fn, EType t, const void* in, void* out, uint64_t n,
 hipError_t launch_mock_prefill(const void* in, void* k, void* v, uint64_t nk, uint64_t nv, hipStream_t s);
 hipError_t launch_rms_norm(EType t, const void* in, const void* w, void* out, uint32_t rows, uint32_t dim, float eps,
                            hipStream_t s);
-// batch: rope_batch ([seq, n_heads, head_dim], pos = token + step); else rope (pos = step).
-hipError_t launch_rope(EType t, bool batch, const void* in, void* out, uint64_t n, uint32_t n_heads,
-                       uint32_t head_dim, uint32_t step, float theta, hipStream_t s);
+// The residual addition and the norm after it: sum = a + b, out = rms_norm of
+// sum; and silu with the product after it: act = silu(gate), out = act * up.
+// The bits of the separate launches; hipErrorNotSupported for operands (odd
+// alignment, row lengths) that need them.
+hipError_t launch_add_rms_norm(EType t, const void* a, const void* b, void* sum, const void* w, void* out,
+                               uint32_t rows, uint32_t dim, float eps, hipStream_t s);
+hipError_t launch_silu_mul(EType t, const void* gate, const void* up, void* act, void* out, uint64_t n, hipStream_t s);
+// batch: rope_batch ([seq, n_heads, head_dim], pos = token + step); else rope
+// (pos = step).  One or two jobs of n elements each in a launch.
+struct RopeArgs {
+  const void* in;
+  void* out;
+  uint64_t n;
+  uint32_t n_heads;
+};
+hipError_t launch_rope(EType t, bool batch, const RopeArgs* jobs, uint32_t n_jobs, uint32_t head_dim, uint32_t step,
+                       float theta, hipStream_t s);
 // ws: the provider workspace (partials of rows split into chunks), may be null
 hipError_t launch_softmax(const void* in, void* out, uint32_t rows, uint32_t dim, float* ws, size_t ws_floats,
                           hipStream_t s);

@@ -603,9 +603,10 @@ hipError_t run_plan(const Plan& pl, Buffer* const* in, Buffer* const* out, int g
     case Path::RmsNorm:
       return launch_rms_norm(pl.c, in[0]->dev, in[1]->dev, out[0]->dev, pl.lp.rows, pl.lp.dim, pl.lp.eps, s);
     case Path::Rope:
-    case Path::RopeBatch:
-      return launch_rope(pl.c, pl.path == Path::RopeBatch, in[0]->dev, out[0]->dev, pl.count, pl.lp.n_heads,
-                         pl.lp.head_dim, pl.lp.step, pl.lp.theta, s);
+    case Path::RopeBatch: {
+      const RopeArgs job{in[0]->dev, out[0]->dev, pl.count, pl.lp.n_heads};
+      return launch_rope(pl.c, pl.path == Path::RopeBatch, &job, 1, pl.lp.head_dim, pl.lp.step, pl.lp.theta, s);
+    }
     case Path::Softmax:
       return launch_softmax(in[0]->dev, out[0]->dev, pl.lp.rows, pl.lp.dim, ws.part, ws.part_floats, s);
     case Path::Embedding:
@@ -710,9 +711,39 @@ bool waits_on_event(const Prepared& pr) {
   return false;
 }
 
+// One launch for a group that groupable() or fusable() accepted;
+// hipErrorNotSupported if the kernel declines it.
+hipError_t run_group(const Prepared* prs, uint32_t n, const Workspace& ws, hipStream_t s) {
+  const Plan& pl = prs[0].pl;
+  const Plan& nx = prs[1].pl;
+  GemvJob jobs[kGemvGroupMax];
+  switch (pl.path) {
+    case Path::Gemv:
+    case Path::Skinny:
+      for (uint32_t j = 0; j < n; ++j) jobs[j] = GemvJob{prs[j].in[1]->dev, prs[j].out[0]->dev, prs[j].pl.N};
+      return pl.path == Path::Gemv ? launch_gemv_group(pl.q, pl.c, prs[0].in[0]->dev, jobs, n, pl.M, pl.K, s)
+                                   : launch_skinny_group(pl.q, pl.c, prs[0].in[0]->dev, jobs, n, pl.M, pl.K, ws, s);
+    case Path::Rope:
+    case Path::RopeBatch: {
+      const RopeArgs rj[2] = {{prs[0].in[0]->dev, prs[0].out[0]->dev, pl.count, pl.lp.n_heads},
+                              {prs[1].in[0]->dev, prs[1].out[0]->dev, nx.count, nx.lp.n_heads}};
+      return launch_rope(pl.c, pl.path == Path::RopeBatch, rj, 2, pl.lp.head_dim, pl.lp.step, pl.lp.theta, s);
+    }
+    case Path::Binary:
+      return launch_add_rms_norm(pl.c, prs[0].in[0]->dev, prs[0].in[1]->dev, prs[0].out[0]->dev, prs[1].in[1]->dev,
+                                 prs[1].out[0]->dev, nx.lp.rows, nx.lp.dim, nx.lp.eps, s);
+    case Path::Unary: {
+      const void* act = prs[0].out[0]->dev;
+      const void* up = prs[1].in[prs[1].in[0]->dev == act ? 1 : 0]->dev;
+      return launch_silu_mul(pl.c, prs[0].in[0]->dev, up, prs[0].out[0]->dev, prs[1].out[0]->dev, pl.count, s);
+    }
+    default: return hipErrorNotSupported;
+  }
+}
+
 // Enqueue prepared dispatches in order.  n > 1 only for a group that
-// groupable() accepted: one grouped launch of the GEMV or small-batch kernel
-// (or, if the kernel declines the group, one launch each).
+// groupable() or fusable() accepted: one launch for it (or, if the kernel
+// declines the group, the first on its own and the rest the same way).
 nf_status launch(Provider* p, const Prepared* prs, uint32_t n) {
   hipError_t e = hipSuccess;
   {
@@ -734,17 +765,8 @@ nf_status launch(Provider* p, const Prepared* prs, uint32_t n) {
     if (n == 1) {
       e = run_plan(prs[0].pl, prs[0].in, prs[0].out, p->tuning.gemm_tile, p->ws, p->stream);
     } else {
-      GemvJob jobs[kGemvGroupMax];
-      for (uint32_t j = 0; j < n; ++j) jobs[j] = GemvJob{prs[j].in[1]->dev, prs[j].out[0]->dev, prs[j].pl.N};
-      const Plan& pl = prs[0].pl;
-      // One launch for the group; if the kernel declines, the first job on
-      // its own and then the rest the same way.
       for (uint32_t j0 = 0; j0 < n && e == hipSuccess;) {
-        e = hipErrorNotSupported;
-        if (n - j0 > 1)
-          e = pl.path == Path::Gemv
-                  ? launch_gemv_group(pl.q, pl.c, prs[0].in[0]->dev, jobs + j0, n - j0, pl.M, pl.K, p->stream)
-                  : launch_skinny_group(pl.q, pl.c, prs[0].in[0]->dev, jobs + j0, n - j0, pl.M, pl.K, p->ws, p->stream);
+        e = n - j0 > 1 ? run_group(prs + j0, n - j0, p->ws, p->stream) : hipErrorNotSupported;
         if (e != hipErrorNotSupported) break;
         if (n - j0 > 1) p->launch_groups.fetch_add(1, std::memory_order_relaxed);
         e = run_plan(prs[j0].pl, prs[j0].in, prs[j0].out, p->tuning.gemm_tile, p->ws, p->stream);
@@ -1137,6 +1159,43 @@ bool groupable(const Prepared* g, uint32_t n, const Prepared& next) {
   return !overlaps(next.out[0], next.in[0]) && !overlaps(next.out[0], next.in[1]);
 }
 
+// Exactly the same memory, or none in common.
+bool same_or_apart(const Buffer* a, const Buffer* b) { return a->dev == b->dev || !overlaps(a, b); }
+
+// Whether `next` right after `a` runs in one launch with it: two ropes of one
+// head_dim, step and theta (a layer's q and k); the residual addition and the
+// norm of its sum; silu and the product with its output.  Every output of
+// both is written, and no buffer written by one overlaps one the other reads
+// or writes except element by element in the same thread, so the result is
+// that of running them in order.
+bool fusable(const Prepared& a, const Prepared& next) {
+  const Plan& p = a.pl;
+  const Plan& q = next.pl;
+  if (p.c != q.c || p.count == 0 || q.count == 0) return false;
+  if (p.path == Path::Rope || p.path == Path::RopeBatch)
+    return q.path == p.path && p.lp.head_dim == q.lp.head_dim && p.lp.step == q.lp.step &&
+           std::memcmp(&p.lp.theta, &q.lp.theta, sizeof(float)) == 0 && !overlaps(next.out[0], a.in[0]) &&
+           !overlaps(next.out[0], a.out[0]) && !overlaps(a.out[0], next.in[0]);
+  if (p.count != q.count) return false;
+  if (p.path == Path::Binary && p.lp.fn == EwFn::Add && q.path == Path::RmsNorm)
+    return next.in[0]->dev == a.out[0]->dev && same_or_apart(a.out[0], a.in[0]) &&
+           same_or_apart(a.out[0], a.in[1]) && !overlaps(a.out[0], next.in[1]) && !overlaps(next.out[0], a.in[0]) &&
+           !overlaps(next.out[0], a.in[1]) && !overlaps(next.out[0], a.out[0]) && !overlaps(next.out[0], next.in[1]);
+  if (p.path == Path::Unary && p.lp.fn == EwFn::Silu && q.path == Path::Binary && q.lp.fn == EwFn::Mul) {
+    const bool first = next.in[0]->dev == a.out[0]->dev;
+    if (!first && next.in[1]->dev != a.out[0]->dev) return false;
+    const Buffer* up = next.in[first ? 1 : 0];
+    return !overlaps(up, a.out[0]) && same_or_apart(a.out[0], a.in[0]) && same_or_apart(next.out[0], a.in[0]) &&
+           same_or_apart(next.out[0], a.out[0]) && same_or_apart(next.out[0], up);
+  }
+  return false;
+}
+
+bool fusable_head(const Plan& p) {
+  return p.path == Path::Rope || p.path == Path::RopeBatch || (p.path == Path::Binary && p.lp.fn == EwFn::Add) ||
+         (p.path == Path::Unary && p.lp.fn == EwFn::Silu);
+}
+
 NF_API nf_status nf_hip_run_tasks(nf_provider self, const nf_task_desc* tasks, uint32_t n_tasks,
                                   uint32_t repeat) {
   Provider* p = as_prov(self);
@@ -1157,6 +1216,13 @@ NF_API nf_status nf_hip_run_tasks(nf_provider self, const nf_task_desc* tasks, u
             !groupable(prs, n, prs[n]))
           break;
         ++n;
+      }
+      if (group && n == 1 && fusable_head(prs[0].pl) && i + 1 < n_tasks) {
+        const nf_task_desc& u = tasks[i + 1];
+        if (prepare(p, u.op_name, u.inputs, u.n_inputs, const_cast<nf_buffer*>(u.outputs), u.n_outputs, &prs[1]) ==
+                NF_OK &&
+            fusable(prs[0], prs[1]))
+          n = 2;
       }
       st = launch(p, prs, n);
       if (st != NF_OK) return st;

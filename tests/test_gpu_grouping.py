@@ -1,5 +1,6 @@
 """nf_hip_run_tasks merges adjacent decode GEMVs and small-batch linears
-that read the same activation buffer (q/k/v, gate/up) into one launch.  Each
+that read the same activation buffer (q/k/v, gate/up) into one launch, and
+pairs of layer ops (two ropes, add and norm, silu and product).  Each
 result must be bit-identical to dispatching the tasks one by one, the launch
 count must show the merge, and a hazard between two tasks (here: both write
 the same output; a weight buffer written mid-list; each task reading the
@@ -208,4 +209,71 @@ def test_run_tasks_dependent_sequence(provider, oracle_mod, fmt, f16, dims):
         assert_close(chained[0].reshape(M, dims[1]).astype(np.float32), ref.astype(np.float32), what=f"{fmt} layer 0")
     finally:
         for b in acts + ws:
+            b.release()
+
+
+# A layer op and the one after it in one launch: per pair, the ops as (op,
+# inputs, output) over named buffers, and the launches expected for rows of a
+# whole number of 16-byte chunks.  "a", "b" and "u" hold data, "w" f32 weights.
+FUSED = {
+    "rope": ([("rope_batch", ["a"], "s"), ("rope_batch", ["b"], "t")], 1),
+    "rope_in_place": ([("rope_batch", ["a"], "a"), ("rope_batch", ["b"], "b")], 1),
+    "rope_chained": ([("rope_batch", ["a"], "s"), ("rope_batch", ["s"], "t")], 2),
+    "rope_silu": ([("rope_batch", ["a"], "s"), ("silu", ["b"], "t")], 2),
+    "add_norm": ([("metal_vector_add", ["a", "b"], "s"), ("rms_norm", ["s", "w"], "t")], 1),
+    "add_norm_residual": ([("metal_vector_add", ["a", "b"], "a"), ("rms_norm", ["a", "w"], "t")], 1),
+    "add_norm_overwrites": ([("metal_vector_add", ["a", "b"], "s"), ("rms_norm", ["s", "w"], "b")], 2),
+    "add_norm_in_place": ([("metal_vector_add", ["a", "b"], "s"), ("rms_norm", ["s", "w"], "s")], 2),
+    "silu_mul": ([("silu", ["a"], "s"), ("elementwise_mul", ["s", "u"], "t")], 1),
+    "silu_mul_swapped": ([("silu", ["a"], "s"), ("elementwise_mul", ["u", "s"], "t")], 1),
+    "silu_mul_in_place": ([("silu", ["a"], "a"), ("elementwise_mul", ["a", "u"], "u")], 1),
+    "silu_mul_onto_gate": ([("silu", ["a"], "s"), ("elementwise_mul", ["s", "u"], "a")], 1),
+    "silu_squared": ([("silu", ["a"], "s"), ("elementwise_mul", ["s", "s"], "t")], 2),
+    "silu_add": ([("silu", ["a"], "s"), ("metal_vector_add", ["s", "u"], "t")], 2),
+}
+
+
+@pytest.mark.parametrize("f16", [False, True], ids=["f32", "f16"])
+@pytest.mark.parametrize("rows,dim", [(1, 64), (3, 2048), (2, 260), (5, 30), (1, 8192), (600, 128)],
+                         ids=lambda v: str(v))
+@pytest.mark.parametrize("pair", sorted(FUSED))
+def test_run_tasks_layer_pairs(provider, pair, rows, dim, f16):
+    """Both outputs bit-identical to one dispatch each, with infinities and
+    NaN among the inputs; rows that are no whole number of 16-byte chunks
+    (260 halves, 30 elements) and operands in the way take two launches.
+    The second rope has fewer heads than the first."""
+    from neurofabric_amd.plugin import push_constants
+    npdt, dt = (np.float16, abi.NF_DTYPE_F16) if f16 else (np.float32, abi.NF_DTYPE_F32)
+    rng = np.random.default_rng(rows * dim + f16)
+    data = {n: rng.standard_normal((rows, dim)).astype(npdt) for n in "abust"}
+    data["a"][0, :3] = np.inf, -np.inf, np.nan
+    data["u"][-1, -1] = -np.inf
+    data["w"] = rng.standard_normal(dim).astype(np.float32)
+    bufs = {n: provider.alloc_array(x, abi.NF_DTYPE_F32 if n == "w" else dt) for n, x in data.items()}
+    steps, launches = FUSED[pair]
+    heads = 2 if rows % 2 == 0 else 1
+    tasks = [provider.task(op, [bufs[n] for n in ins], [bufs[out]],
+                           pc=push_constants(seq_len=rows, n_heads=heads if i == 0 else 1, head_dim=dim, epsilon=1e-5,
+                                             theta=10000.0, step_idx=7))
+             for i, (op, ins, out) in enumerate(steps)]
+    if not pair.startswith("rope"):
+        per = 8 if f16 else 4
+        # the norm needs whole chunks of a row, silu and mul only aligned buffers
+        if pair.startswith("add") and dim % per:
+            launches = 2
+    try:
+        before = provider.launch_count()
+        provider.run_tasks(_array(tasks), 1)
+        provider.synchronize()
+        assert provider.launch_count() - before == launches
+        got = {n: b.download(data[n].dtype).copy() for n, b in bufs.items()}
+        for n, b in bufs.items():
+            b.upload(data[n])
+        for td in tasks:
+            provider.check(provider.dispatch_task(td), "dispatch")
+        provider.synchronize()
+        for n, b in bufs.items():
+            assert np.array_equal(got[n].view(np.uint8), b.download(data[n].dtype).view(np.uint8)), n
+    finally:
+        for b in bufs.values():
             b.release()
