@@ -1073,6 +1073,50 @@ __global__ __launch_bounds__(256) void append_kernel(const T* __restrict__ kn, c
   cv[dst] = vn[id];
 }
 
+// The same copy in 16-byte chunks (row_chunks a row; the launcher sees to the
+// alignment and to counts below 2^32).  The element-wise kernel is bound by
+// its address arithmetic, two 64-bit divisions per element; here a chunk takes
+// two 32-bit ones.  2048 tokens of 8 KV heads x 128 f16, the whole attention
+// dispatch: 84.3 -> 82.1 us.
+template <bool HEAD_MAJOR>
+__global__ __launch_bounds__(256) void append_vec_kernel(const u32x4* __restrict__ kn, const u32x4* __restrict__ vn,
+                                                         u32x4* __restrict__ ck, u32x4* __restrict__ cv,
+                                                         uint32_t n, uint32_t n_kv, uint32_t tokens,
+                                                         uint32_t row_chunks, uint32_t max_seq, uint32_t first_pos) {
+  const uint32_t id = blockIdx.x * 256 + threadIdx.x;
+  if (id >= n) return;
+  const u32x4 k = kn[id], v = vn[id];
+  const uint32_t row = id / row_chunks, c = id - row * row_chunks;
+  const uint32_t div = HEAD_MAJOR ? tokens : n_kv;
+  const uint32_t hi = row / div, lo = row - hi * div;
+  const uint32_t kvh = HEAD_MAJOR ? hi : lo, tok = HEAD_MAJOR ? lo : hi;
+  const uint64_t dst = ((uint64_t)kvh * max_seq + first_pos + tok) * row_chunks + c;
+  ck[dst] = k;
+  cv[dst] = v;
+}
+
+template <typename T>
+hipError_t launch_append(bool head_major, const void* kn, const void* vn, void* ck, void* cv, uint32_t n_kv,
+                         uint32_t tokens, uint32_t dim, uint32_t max_seq, uint32_t first_pos, hipStream_t s) {
+  const uint64_t n = (uint64_t)n_kv * tokens * dim;
+  const bool al16 = ((reinterpret_cast<uintptr_t>(kn) | reinterpret_cast<uintptr_t>(vn) |
+                      reinterpret_cast<uintptr_t>(ck) | reinterpret_cast<uintptr_t>(cv)) & 15) == 0;
+  constexpr uint32_t V = 16 / sizeof(T);
+  // whole chunks per row and aligned rows; past 2^31 chunks (32 GiB) the
+  // kernel's 32-bit index would end
+  if (al16 && dim % V == 0 && n / V <= (1ull << 31)) {
+    const uint32_t nc = (uint32_t)(n / V);
+    auto* kernel = head_major ? append_vec_kernel<true> : append_vec_kernel<false>;
+    kernel<<<dim3((nc + 255) / 256), 256, 0, s>>>((const u32x4*)kn, (const u32x4*)vn, (u32x4*)ck, (u32x4*)cv, nc, n_kv,
+                                                  tokens, dim / V, max_seq, first_pos);
+  } else {
+    auto* kernel = head_major ? append_kernel<T, true> : append_kernel<T, false>;
+    kernel<<<dim3((unsigned)((n + 255) / 256)), 256, 0, s>>>((const T*)kn, (const T*)vn, (T*)ck, (T*)cv, n_kv, tokens,
+                                                             dim, max_seq, first_pos);
+  }
+  return hipGetLastError();
+}
+
 // ---- decode: split the keys over many workgroups ----------------------------------
 //
 // One query token per head, so the work is the KV cache read.  Workgroup =
@@ -1746,11 +1790,8 @@ hipError_t run(const Params& p, uint32_t nq, float* ws, size_t ws_floats, hipStr
     const hipError_t e = run_decode_split<T, MODE>(p, ws, ws_floats, s);
     if (e != hipErrorNotSupported) return e;
     if (p.fused_append) {  // the split kernel declined: append here first
-      const uint64_t n = (uint64_t)p.n_kv * p.dim;
-      append_kernel<T, MODE == nfhip::AttnMode::Gqa><<<(unsigned)((n + 255) / 256), 256, 0, s>>>(
-          static_cast<const T*>(p.k_new), static_cast<const T*>(p.v_new), static_cast<T*>(p.k),
-          static_cast<T*>(p.v), p.n_kv, 1, p.dim, p.max_seq, p.step);
-      const hipError_t e2 = hipGetLastError();
+      const hipError_t e2 = launch_append<T>(MODE == nfhip::AttnMode::Gqa, p.k_new, p.v_new, p.k, p.v, p.n_kv, 1,
+                                             p.dim, p.max_seq, p.step, s);
       if (e2 != hipSuccess) return e2;
     }
   }
@@ -1807,16 +1848,8 @@ hipError_t launch_t(const nfhip::AttnArgs& a, hipStream_t s) {
   const bool fuse = lp.append && lp.decode && a.ws != nullptr;
   if (lp.append && !fuse) {
     const uint32_t tokens = lp.decode ? 1 : lp.seq_len;
-    const uint64_t n = (uint64_t)lp.n_kv * tokens * lp.head_dim;
-    const dim3 grid((unsigned)((n + 255) / 256));
-    const uint32_t first = lp.decode ? lp.step : 0;
-    if (lp.attn == nfhip::AttnMode::Gqa)
-      append_kernel<T, true><<<grid, 256, 0, s>>>((const T*)a.k_new, (const T*)a.v_new, (T*)a.k, (T*)a.v, lp.n_kv,
-                                                  tokens, lp.head_dim, lp.max_seq, first);
-    else
-      append_kernel<T, false><<<grid, 256, 0, s>>>((const T*)a.k_new, (const T*)a.v_new, (T*)a.k, (T*)a.v, lp.n_kv,
-                                                   tokens, lp.head_dim, lp.max_seq, first);
-    hipError_t e = hipGetLastError();
+    const hipError_t e = launch_append<T>(lp.attn == nfhip::AttnMode::Gqa, a.k_new, a.v_new, a.k, a.v, lp.n_kv, tokens,
+                                          lp.head_dim, lp.max_seq, lp.decode ? lp.step : 0, s);
     if (e != hipSuccess) return e;
   }
   Params p{};

@@ -351,6 +351,17 @@ def test_attention(provider, op, f16, kw):
         assert np.array_equal(gk, wk) and np.array_equal(gv, wv), "cache append"
 
 
+# Rows appended in 16-byte chunks (rows of 1, 5, 16 and 24 chunks, a last
+# workgroup that is partly empty) and, where a row is no whole number of
+# them, element by element; both source orders.  Copies, so exact.
+@pytest.mark.parametrize("op", ["flash_attention_cached", "flash_attention_gqa"])
+@pytest.mark.parametrize("f16,D", [(False, 4), (True, 40), (False, 64), (True, 192), (True, 36), (False, 6)])
+@pytest.mark.parametrize("S", [1, 37])
+def test_attention_append(provider, op, f16, D, S):
+    _, _, (gk, gv, wk, wv) = _attn_case(provider, op, f16, H=6, KV=3, D=D, S=S, step=0, max_seq=41, seed=D + S)
+    assert np.array_equal(gk, wk) and np.array_equal(gv, wv)
+
+
 @pytest.mark.parametrize("op,kw,bad,f16", [
     ("causal_attention", dict(H=4, KV=4, D=64, S=50, step=0, max_seq=0), 40, False),
     ("flash_attention_cached", dict(H=4, KV=4, D=128, S=130, step=0, max_seq=160, window=40), 10, False),
