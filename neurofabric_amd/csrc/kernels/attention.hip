@@ -1397,7 +1397,13 @@ __global__ __launch_bounds__(64) void decode_split_kernel(Params p, uint32_t key
 //    together with the keys, and takes the tile's weights from LDS;
 //  * the NW waves' (m, l, acc) are merged in LDS and written as the split's
 //    partial (m in natural-log units); decode_combine_kernel adds the
-//    splits.
+//    splits.  A lone split (up to 128 keys) writes the output itself and no
+//    second kernel runs: 32 heads over 4 KV heads x 64, f32, 61 / 128 keys,
+//    8.0 / 8.3 -> 5.7 / 5.9 us; over 8 x 128, f16, 7.7 / 7.9 -> 5.2 / 5.4.
+//    (Measured and not kept: lone splits of 8 waves up to 256 keys, 8.2 ->
+//    7.7 us at the first shape but 9.7 -> 10.5 at 8 x 128 f32, and of 16
+//    waves up to 512 keys, 8.2 -> 12.3: one CU's read of a KV head's cache
+//    takes longer than the second launch.)
 //    (Measured and not kept: the merge in the last-arriving workgroup of
 //    each KV head, 15.7 against 11.4 us at 4096 keys: the store, counter
 //    and reload round trips cost more than a second launch; a one-pass
@@ -1611,7 +1617,7 @@ __global__ __launch_bounds__(NW * 64) void decode_mfma_kernel(Params p, uint32_t
   }
   __syncthreads();
 
-  // ---- merge the 4 waves and write the split's partial per head -----------------
+  // ---- merge the waves; write the split's partial per head, or the output -------
   const uint32_t stride = D + 2;
   for (int idx = tid; idx < ng * DD; idx += NT) {
     const int g = idx / DD, d = idx % DD;
@@ -1624,6 +1630,10 @@ __global__ __launch_bounds__(NW * 64) void decode_mfma_kernel(Params p, uint32_t
       const float f = wm[v][g] == -INFINITY ? 0.f : exp2f(wm[v][g] - M);
       L += f * wl[v][g];
       A += f * wacc[v][g][d];
+    }
+    if (!part) {  // the only split
+      static_cast<T*>(p.out)[q_row<MODE>(p, 0, 0) + (uint64_t)(h0 + g) * D + d] = (T)(A * (L > 0.f ? 1.0f / L : 0.f));
+      continue;
     }
     float* dst = part + ((uint64_t)split * H + h0 + g) * stride;
     if (d == 0) {
@@ -1750,16 +1760,32 @@ hipError_t run_decode_split(const Params& p, float* ws, size_t ws_floats, hipStr
       const uint64_t ns = (n_keys + 4 * tk - 1) / (4 * tk);
       if (ns <= (uint64_t)kMaxSplits && ns * H * (p.dim + 2) <= ws_floats) {
         const dim3 g2((unsigned)ns, KV);
+        // one split writes the output, unless that lies in memory other
+        // workgroups still read (the same buffer as the query is fine: each
+        // workgroup reads only the heads it writes)
+        const uint64_t rows = MODE == nfhip::AttnMode::Paged ? p.pool_blocks * p.block_size : p.max_seq;
+        const uint64_t cache = rows * KV * p.dim * sizeof(T), fresh = p.fused_append ? (uint64_t)KV * p.dim * sizeof(T) : 0;
+        const T* o = static_cast<const T*>(p.out) + q_row<MODE>(p, 0, 0);
+        const T* qr = static_cast<const T*>(p.q) + q_row<MODE>(p, 0, 0);
+        const uint64_t ob = (uint64_t)H * p.dim * sizeof(T);
+        auto apart = [&](const void* m, uint64_t bytes) {
+          const uintptr_t a = reinterpret_cast<uintptr_t>(o), b = reinterpret_cast<uintptr_t>(m);
+          return a + ob <= b || b + bytes <= a;
+        };
+        const bool alone = ns == 1 && (o == qr || apart(qr, ob)) && apart(p.k, cache) && apart(p.v, cache) &&
+                           apart(p.k_new, fresh) && apart(p.v_new, fresh) &&
+                           apart(p.table, MODE == nfhip::AttnMode::Paged ? p.n_blocks * sizeof(uint32_t) : 0);
+        float* part = alone ? nullptr : ws;
 #define NF_DECODE_MFMA(DDD, GG)                                                                      \
   if (p.dim == DDD && G == GG) {                                                                     \
-    if (tk == 32) decode_mfma_kernel<T, MODE, DDD, GG, 32, 4><<<g2, 256, 0, s>>>(p, 4 * tk, lo, ws);  \
-    else decode_mfma_kernel<T, MODE, DDD, GG, 64, 4><<<g2, 256, 0, s>>>(p, 4 * tk, lo, ws);           \
+    if (tk == 32) decode_mfma_kernel<T, MODE, DDD, GG, 32, 4><<<g2, 256, 0, s>>>(p, 4 * tk, lo, part);  \
+    else decode_mfma_kernel<T, MODE, DDD, GG, 64, 4><<<g2, 256, 0, s>>>(p, 4 * tk, lo, part);           \
   }
         NF_DECODE_MFMA(64, 1) NF_DECODE_MFMA(64, 2) NF_DECODE_MFMA(64, 4) NF_DECODE_MFMA(64, 8)
         NF_DECODE_MFMA(128, 1) NF_DECODE_MFMA(128, 2) NF_DECODE_MFMA(128, 4) NF_DECODE_MFMA(128, 8)
 #undef NF_DECODE_MFMA
         hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
+        if (e != hipSuccess || !part) return e;
         decode_combine_kernel<T><<<dim3(H, (p.dim + 31) / 32), 1024, 0, s>>>(ws, (uint32_t)ns, H, p.dim, static_cast<T*>(p.out),
                                                    q_row<MODE>(p, 0, 0), p.dim);
         return hipGetLastError();

@@ -362,6 +362,24 @@ def test_attention_append(provider, op, f16, D, S):
     assert np.array_equal(gk, wk) and np.array_equal(gv, wv)
 
 
+# Decode around the contexts one workgroup per KV head takes whole and
+# finishes itself (up to 128 keys): 2 keys, one short of it, just full, one
+# key past it, windows on both sides of it, groups of 1, 3 and 8 heads.  fp32
+# sums in another order: the bounds of test_attention.
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("H,KV,D", [(8, 1, 64), (6, 2, 64), (4, 4, 128), (8, 1, 128)])
+@pytest.mark.parametrize("keys,window", [(2, 0), (127, 0), (128, 0), (129, 0), (600, 128), (600, 129)])
+@pytest.mark.parametrize("op", ["flash_attention_cached", "flash_attention_gqa"])
+def test_decode_split_edges(provider, op, f16, H, KV, D, keys, window):
+    got, want, (gk, gv, wk, wv) = _attn_case(provider, op, f16, H=H, KV=KV, D=D, S=1, step=keys - 1, max_seq=600,
+                                             window=window, seed=keys + D)
+    if f16:
+        assert _ulp16_ok(got, want, ulps=2, abs_frac=1e-5)
+    else:
+        assert np.max(np.abs(got - want)) <= 2e-5 * np.max(np.abs(want))
+    assert np.array_equal(gk, wk) and np.array_equal(gv, wv)
+
+
 @pytest.mark.parametrize("op,kw,bad,f16", [
     ("causal_attention", dict(H=4, KV=4, D=64, S=50, step=0, max_seq=0), 40, False),
     ("flash_attention_cached", dict(H=4, KV=4, D=128, S=130, step=0, max_seq=160, window=40), 10, False),
