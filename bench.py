@@ -420,7 +420,7 @@ def crossover_sweep(prov, shapes=((28672, 8192), (8192, 28672)), Ms=(1, 2, 4, 8,
     """the Llama-70B FFN gate/up (28672x8192) and down
     (8192x28672) Q4_0 projections, f16 activations, through every kernel
     family that serves each M (switch points pinned): the VALU GEMV (while
-    its activation stage fits in LDS), the small-batch MFMA kernel (M <= 64,
+    its activation stage fits in LDS), the small-batch MFMA kernel (M <= 128,
     one launch) and the tiled MFMA GEMM.  Each measurement replays (graph)
     `copies` launches over distinct copies of the weights (4 x 132 MB, twice
     the Infinity Cache), 5 times; the weights are uploaded once per shape."""
@@ -450,7 +450,7 @@ def crossover_sweep(prov, shapes=((28672, 8192), (8192, 28672)), Ms=(1, 2, 4, 8,
                         st.add("dequant_q4_0_linear_f16", [a, w], [c], M, N, K)
                     st.finish()
                     kern = sorted(st.kernels)[0]
-                    if not kern.startswith(family[path]) or (path == "skinny" and M > 64):
+                    if not kern.startswith(family[path]) or (path == "skinny" and M > 128):
                         continue  # this family does not serve M here
                     r = time_step(prov, st, 5, 2, "graph")
                     us = r["us_per_launch"]

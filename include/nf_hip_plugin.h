@@ -115,7 +115,10 @@ NF_API nf_status nf_hip_plan_dispatch(const char *op_name,
  * launch), the tiled MFMA GEMM beyond (f16 activations: fp16 MFMA; f32
  * activations: exact bf16 pieces on bf16 MFMA, K % 64 == 0).  f16 and f32
  * activations each have their own switch points.  Defaults come from
- * measurement; environment overrides NF_HIP_GEMV_MAX_M_F32,
+ * measurement; the f16 default of skinny_max_m, 128, leaves batches of 17 to
+ * 128 rows to the tiled GEMM where that measured faster or a GEMM kernel is
+ * forced (nf_hip_set_gemm_tile), any other value is taken as it stands.
+ * Environment overrides NF_HIP_GEMV_MAX_M_F32,
  * NF_HIP_GEMV_MAX_M_F16, NF_HIP_SKINNY_MAX_M_F16 and NF_HIP_SKINNY_MAX_M_F32
  * are read at nf_plugin_register.  No counterpart in the reference: its
  * Metal provider runs one kernel for every M (metal_provider.mm:3009-3019,

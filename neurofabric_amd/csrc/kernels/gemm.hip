@@ -1967,18 +1967,6 @@ hipError_t launch_gemm_mfma(QFmt q, EType t, const void* A, const void* W, void*
     // one-wave kernel, tiles 8 / 9 / 10 the two-wave kernel with 128 / 64 /
     // 32-row waves (8: Q4_0 only), tile 11 the 128-row waves on 128 x 128
     // tiles (Q4_0 only); 0..6 select one of the LDS-staged tile shapes.
-    //
-    // Up to 128 rows the small-batch kernel (skinny.hip) is the faster one
-    // wherever it takes the operands (K % 256 == 0): us, these kernels ->
-    // that one, 8192x28672 Q4_0 M = 32 / 64 61.5 / 71.9 -> 43 / 56,
-    // 4096x4096 Q8_0 M = 32 / 64 / 128 23.4 / 30.4 / 29.6 -> 9.0 / 11.4 /
-    // 17.6, 14336x4096 Q4_0 M = 128 34.9 -> 32.8; but not above 64 rows of
-    // Q4_0 past about 88 M weights, where it is bound by its MFMA operand
-    // reads (32000x4096 M = 128 55.0 against 63.1, 28672x8192 91.0 against
-    // 115; Q8_0 there 71.3 against 61.6 and 114 against 107).
-    if (tile < 0 && skinny_fits(M, N, K, A, W) &&
-        (M <= 64 || q == QFmt::Q8_0 || (uint64_t)N * K <= (88ull << 20)))
-      return launch_skinny(q, t, A, W, C, M, N, K, ws, s);
     const bool k128 = K % 128 == 0;
     const bool q4 = q == QFmt::Q4_0;
     const long tiles64 = (long)((M + 63) / 64) * (long)((N + 255) / 256);

@@ -93,6 +93,33 @@ nf_status read_mnk(const uint8_t* pc, uint32_t pc_size, uint32_t* M, uint32_t* N
   return NF_OK;
 }
 
+// Whether an f16 batch of 17 to 128 rows runs faster on the small-batch kernel
+// than on the tiled GEMM.  The lines lie where the small-batch kernel's row
+// tiles (64, 128 or 256 weight rows by batch and format) need a second round
+// of workgroups, past which a launch reads its activations again and the
+// tiled kernel's few large tiles win.  Measured on MI355X, us per launch over
+// rotated weights, tiled / small-batch:
+//   up to 32 rows    always: Q4_0 32000x2048 M = 32 22.5 / 15.1, Q8_0
+//                    28672x8192 100 / 72; at worst 40960x256 7.8 / 8.0
+//   33 to 64 rows    N <= 32768: Q4_0 32000x2048 M = 64 28.5 / 20.0; above,
+//                    Q4_0 65536x768 18.6 / 21.9 but 65536x4096 72.4 / 66.6,
+//                    Q8_0 65536x768 26.3 / 29.5 but 65536x2048 61.8 / 55.6
+//   65 to 128 rows   Q4_0 N <= 16384: 16384x2048 M = 128 x 0.76, 20480x2048
+//                    27.7 / 32.4, 32000x2048 30.9 / 34.6, and up to 88 M
+//                    weights: 8192x28672 93.0 / 110.7; Q8_0 N <= 32768:
+//                    32000x2048 48.6 / 37.4, 65536x2048 62.6 / 72.6
+// The tiled kernel stores its output element by element where N is no
+// multiple of 4, so there the small-batch kernel stays ahead for longer:
+// 50257x768 Q4_0 M = 64 / 128 24.2 / 20.8 and 43.1 / 35.8, 50256x768 16.5 /
+// 20.5 and 30.8 / 35.1.
+bool skinny_f16_faster(QFmt q, uint32_t M, uint32_t N, uint32_t K) {
+  const bool q4 = q == QFmt::Q4_0, split_stores = N % 4 != 0;
+  if (M <= 32) return true;
+  if (M <= 64) return split_stores || N <= 32768 || K >= (q4 ? 4096u : 1536u);
+  if (N <= (q4 ? 16384u : 32768u)) return !q4 || (uint64_t)N * K <= (88ull << 20);
+  return split_stores && K <= 2048;
+}
+
 }  // namespace
 
 bool op_known(const char* op_name) {
@@ -195,7 +222,9 @@ nf_status make_plan(const char* op_name, const nf_tensor_desc* const* ins, uint3
         p.path = Path::Gemv;
         p.kernel = "gemv_" + tag;
       } else if (K % 256 == 0 && p.M <= (f16 ? tuning.skinny_max_m_f16 : tuning.skinny_max_m_f32) &&
-                 (!f16 || p.M <= 4 || K <= tuning.skinny_f16_max_k)) {
+                 (!f16 || p.M <= 4 || K <= tuning.skinny_f16_max_k) &&
+                 (!f16 || p.M <= 16 || tuning.skinny_max_m_f16 != kSkinnyMaxMF16 ||
+                  (tuning.gemm_tile < 0 && skinny_f16_faster(p.q, p.M, p.N, p.K)))) {
         p.path = Path::Skinny;
         p.kernel = "skinny_mfma_" + tag;
       } else if (f16 || K % 64 == 0) {

@@ -73,8 +73,9 @@ struct LayerParams {
 // Switch points between the kernel families of the fused op: the VALU GEMV
 // while M <= gemv_max_m (and its activation stage fits in LDS), the
 // small-batch MFMA kernel while M <= skinny_max_m (f16 and f32 activations
-// each have their own), the tiled MFMA GEMM above (f16: fp16 MFMA, whose
-// launcher leaves batches up to 64 or 128 rows to the small-batch kernel; f32: bf16-piece MFMA, K % 64 == 0, else the GEMV).
+// each have their own), the tiled MFMA GEMM above (f16: fp16 MFMA; f32:
+// bf16-piece MFMA, K % 64 == 0, else the GEMV).  For f16 the default
+// skinny_max_m is no plain switch point: see skinny_f16_faster() in plan.cpp.
 // Defaults from measured sweeps on MI355X (graph replay over 4 rotated weight
 // copies).  bench.py's configs[4] section (28672x8192 and 8192x28672 Q4_0,
 // f16 activations): the GEMV is fastest up to M = 2 (31.0 / 38.8 us against
@@ -99,10 +100,11 @@ struct LayerParams {
 // kernel (longer K goes to the tiled GEMM); no cap by default, since the
 // small-batch kernel's K split over workgroups makes it the
 // faster one at K = 28672 too (M = 8: 52.8 against 68.1 us).
+constexpr uint32_t kSkinnyMaxMF16 = 128;  // the rows of one launch
 struct Tuning {
   uint32_t gemv_max_m_f32 = 4;
   uint32_t gemv_max_m_f16 = 4;
-  uint32_t skinny_max_m_f16 = 16;
+  uint32_t skinny_max_m_f16 = kSkinnyMaxMF16;
   uint32_t skinny_max_m_f32 = 64;
   uint64_t gemv_m4_max_weight_bytes = 16ull << 20;
   uint32_t gemv_m2_max_stage_bytes = 80 * 1024;

@@ -181,7 +181,7 @@ def test_config4_selected_kernel(provider, oracle_mod, weights, M, NK):
 
 # (family, M) pairs where the forced family actually serves the shape: the
 # GEMV needs its activation stage (M' x K fp16) within 120 KB of LDS, the
-# small-batch kernel takes any M (64 rows per launch), the tiled GEMM any M.
+# small-batch kernel takes any M (128 rows per launch), the tiled GEMM any M.
 C4_FORCED = [("gemv", 1), ("gemv", 2), ("skinny", 1), ("skinny", 8), ("skinny", 64), ("skinny", 128),
              ("tiled", 1), ("tiled", 16), ("tiled", 64), ("tiled", 256)]
 

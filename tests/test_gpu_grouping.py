@@ -84,6 +84,52 @@ def test_run_tasks_merges_same_input_gemvs(provider, oracle_mod, fmt, f16, M):
             b.release()
 
 
+def _merged_and_apart(provider, fmt, f16, M, Ns, K, seed=0):
+    """Linears of `Ns` weight rows over one activation buffer, as a list and
+    then one dispatch each: (launches of the list, outputs equal bit for
+    bit, the inputs, weights and outputs)."""
+    npdt, dt = (np.float16, abi.NF_DTYPE_F16) if f16 else (np.float32, abi.NF_DTYPE_F32)
+    op = f"dequant_{fmt}_linear" + ("_f16" if f16 else "")
+    A = syn.activations(M, K, seed=seed + M, dtype=npdt)
+    Ws = [syn.weights(fmt, N, K, seed=seed + i) for i, N in enumerate(Ns)]
+    a = provider.alloc_array(A, dt)
+    ws = [provider.alloc_array(W, QDT[fmt]) for W in Ws]
+    cs = [provider.alloc(dt, M * N * A.itemsize) for N in Ns]
+    try:
+        arr = _array([provider.task(op, [a, w], [c], M, N, K) for w, c, N in zip(ws, cs, Ns)])
+        before = provider.launch_count()
+        provider.run_tasks(arr, 2)  # twice: the split-K counters must be back at zero
+        provider.synchronize()
+        launches = provider.launch_count() - before
+        assert launches % 2 == 0
+        merged = [c.download(npdt).copy() for c in cs]
+        for w, c, N in zip(ws, cs, Ns):
+            provider.dispatch(op, [a, w], [c], M, N, K)
+        provider.synchronize()
+        single = [c.download(npdt).copy() for c in cs]
+    finally:
+        for b in [a] + ws + cs:
+            b.release()
+    equal = [np.array_equal(x.view(np.uint8), y.view(np.uint8)) for x, y in zip(merged, single)]
+    return launches // 2, equal, A, Ws, [x.reshape(M, N) for x, N in zip(merged, Ns)]
+
+
+@pytest.mark.parametrize("fmt", ["q4_0", "q8_0"])
+@pytest.mark.parametrize("M", [24, 48, 100])
+@pytest.mark.parametrize("Ns,K", [((640, 640, 640), 1024), ((2048, 256, 256), 2048), ((1500, 1500), 768)],
+                         ids=["qkv", "gqa", "gate_up"])
+def test_run_tasks_merges_f16_batches(provider, oracle_mod, fmt, M, Ns, K):
+    """f16 batches past 16 rows are small-batch launches by default, so lists
+    merge them too; every output has the bits of its own dispatch.  Equal
+    linears always share a launch (one variant and K split)."""
+    launches, equal, A, Ws, out = _merged_and_apart(provider, fmt, True, M, Ns, K, seed=K)
+    assert all(equal), equal
+    assert launches == 1 if len(set(Ns)) == 1 else launches <= len(Ns)
+    for W, N, c in zip(Ws, Ns, out):
+        ref = oracle_mod.fused(A, W, fmt, M, N, K, f16=True, threads=8).view(np.float16)
+        assert_close(c.astype(np.float32), ref.astype(np.float32), what=f"{fmt} {M}x{N}x{K}")
+
+
 def test_run_tasks_keeps_hazards_apart(provider, oracle_mod):
     """Two GEMVs over the same activations that write the same output are
     not merged; the output is the second one's, as in dispatch order."""

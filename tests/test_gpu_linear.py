@@ -131,6 +131,29 @@ def test_kernel_paths_agree(provider, oracle_mod, fmt, f16, M):
 
 
 @pytest.mark.parametrize("fmt", ["q4_0", "q8_0"])
+@pytest.mark.parametrize("M,N,K,tile", [(17, 392, 1024, 10), (32, 257, 1152, 10), (33, 392, 1024, 9),
+                                        (64, 4100, 1152, 9), (100, 392, 1024, 9)])
+def test_small_f16_batches_on_the_tiled_kernels(provider, oracle_mod, fmt, M, N, K, tile):
+    """f16 batches of 17 to 128 rows with the small-batch kernel switched off,
+    or where it does not take them (K % 256 != 0): the two-wave tiled kernels,
+    shown by the bits of the same kernel forced by tile."""
+    old = provider.get_tuning()
+    W = syn.weights(fmt, N, K, seed=N)
+    A = syn.activations(M, K, seed=M, dtype=np.float16)
+    ref = oracle_mod.fused(A, W, fmt, M, N, K, f16=True, threads=8).view(np.float16)
+    try:
+        if K % 256 == 0:
+            _force_path(provider, "tiled", True)
+        got = run_fused(provider, fmt, A, W, M, N, K, True)
+        provider.set_gemm_tile(tile)
+        forced = run_fused(provider, fmt, A, W, M, N, K, True)
+        assert np.array_equal(got.view(np.uint16), forced.view(np.uint16))
+        assert_close(got.astype(np.float32), ref.astype(np.float32), what=f"{fmt} {M}x{N}x{K}")
+    finally:
+        provider.set_tuning(old)
+
+
+@pytest.mark.parametrize("fmt", ["q4_0", "q8_0"])
 @pytest.mark.parametrize("f16", [False, True], ids=["f32", "f16"])
 @pytest.mark.parametrize("shape", [(2, 200, 256), (8, 1000, 768), (16, 64, 4096), (17, 257, 2048),
                                    (33, 130, 512), (64, 96, 1024), (130, 72, 256), (5, 40, 192)],

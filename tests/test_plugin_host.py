@@ -283,8 +283,9 @@ def test_crossover_setter_roundtrip():
 def test_default_switch_points(lib):
     """Defaults from the measured sweeps: GEMV for M <= 4 while its
     activation stage fits in 120 KB of LDS (M = 3..4 only for weights up to
-    16 MB), the small-batch MFMA kernel up to 16 rows, the tiled GEMM beyond
-    (f16); for f32 activations the small-batch kernel up to 64 rows."""
+    16 MB), the small-batch MFMA kernel up to 16 rows, and up to 128 where
+    it measured faster than the tiled GEMM (f16: test_f16_batch_route); for
+    f32 activations the small-batch kernel up to 64 rows."""
     f16 = dict(a=abi.NF_DTYPE_F16, c=abi.NF_DTYPE_F16, op="dequant_q4_0_linear_f16")
     assert _fused(lib, 2, 28672, 8192, **f16)["kernel"] == "gemv_q4_0_f16"   # 2 x 8192 x 2 B = 32 KB
     # M = 2: the GEMV while two of its workgroups fit a CU (stage <= 80 KB)
@@ -303,8 +304,9 @@ def test_default_switch_points(lib):
     # f16, long rows: the small-batch kernel too (no K cap by default)
     assert _fused(lib, 8, 8192, 28672, **f16)["kernel"] == "skinny_mfma_q4_0_f16"
     assert _fused(lib, 16, 8192, 28672, **f16)["kernel"] == "skinny_mfma_q4_0_f16"
-    assert _fused(lib, 17, 28672, 8192, **f16)["kernel"] == "gemm_mfma_q4_0_f16"
-    assert _fused(lib, 32, 8192, 28672, **f16)["kernel"] == "gemm_mfma_q4_0_f16"
+    assert _fused(lib, 17, 28672, 8192, **f16)["kernel"] == "skinny_mfma_q4_0_f16"
+    assert _fused(lib, 32, 8192, 28672, **f16)["kernel"] == "skinny_mfma_q4_0_f16"
+    assert _fused(lib, 129, 8192, 4096, **f16)["kernel"] == "gemm_mfma_q4_0_f16"
     assert _fused(lib, 4, 4096, 4096)["kernel"] == "gemv_q4_0_f32"
     assert _fused(lib, 2, 28672, 8192)["kernel"] == "gemv_q4_0_f32"           # 2 x 8192 x 4 B + sums
     assert _fused(lib, 3, 28672, 8192)["kernel"] == "skinny_mfma_q4_0_f32"    # 4 x 8192 x 4 B > 120 KB
@@ -315,6 +317,42 @@ def test_default_switch_points(lib):
     assert _fused(lib, 65, 14336, 4096, op="dequant_q8_0_linear", bs=34)["kernel"] == "gemm_mfma_q8_0_f32"
     assert _fused(lib, 512, 4096, 11008)["kernel"] == "gemm_mfma_q4_0_f32"
     assert _fused(lib, 100, 64, 96)["kernel"] == "gemv_q4_0_f32"  # K % 64 != 0
+
+
+@pytest.mark.parametrize("q,M,N,K,small", [
+    ("q4_0", 32, 128256, 256, True), ("q8_0", 32, 28672, 8192, True), ("q4_0", 32, 4096, 128, False),
+    ("q4_0", 64, 32768, 768, True), ("q4_0", 64, 32772, 768, False), ("q4_0", 33, 65536, 4096, True),
+    ("q8_0", 64, 65536, 1280, False), ("q8_0", 64, 65536, 1536, True), ("q4_0", 64, 50257, 768, True),
+    ("q4_0", 65, 16384, 4096, True), ("q4_0", 65, 16388, 4096, False), ("q4_0", 128, 8192, 28672, False),
+    ("q8_0", 128, 8192, 28672, True), ("q8_0", 128, 32768, 2048, True), ("q8_0", 128, 32772, 2048, False),
+    ("q4_0", 128, 50257, 2048, True), ("q4_0", 128, 50257, 2304, False), ("q8_0", 129, 4096, 4096, False),
+], ids=lambda v: str(v))
+def test_f16_batch_route(q, M, N, K, small):
+    """f16 batches of 17 to 128 rows by default: the small-batch kernel where
+    it measured faster, under the name of the kernel that runs.  A lower
+    switch point, the K cap or a forced GEMM kernel sends them to the tiled
+    GEMM, a higher switch point to the small-batch kernel."""
+    prov = Provider()
+    kw = dict(a=abi.NF_DTYPE_F16, c=abi.NF_DTYPE_F16, op=f"dequant_{q}_linear_f16", bs=18 if q == "q4_0" else 34)
+    names = {True: f"skinny_mfma_{q}_f16", False: f"gemm_mfma_{q}_f16"}
+    kernel = lambda: _fused(prov.lib, M, N, K, **kw)["kernel"]
+    old = prov.get_tuning()
+    try:
+        assert kernel() == names[small]
+        prov.set_gemm_tile(9)
+        assert kernel() == names[False]
+        prov.set_tuning(old)
+        prov.set_skinny_max_m(old[1], None, K - 1)
+        assert kernel() == names[False]
+        prov.set_tuning(old)
+        for below in (0, 16, M - 1):
+            prov.set_skinny_max_m(below)
+            assert kernel() == names[False], below
+        prov.set_skinny_max_m(1 << 30)
+        assert kernel() == names[K % 256 == 0]
+    finally:
+        prov.set_tuning(old)
+    assert kernel() == names[small]
 
 
 def test_gemv_row_limits(lib):
