@@ -566,7 +566,7 @@ float sk_cost(const SkJobs& jobs, uint32_t K) {
 // A launch's variant (index into sk_variants' list for its MT), the order of
 // its sums (GN and NB) and its K split.
 struct SkPick {
-  float key = 1e30f, cost = 1e30f;
+  float key = 1e30f;
   int variant = -1, order = 0, kg = 1;
 };
 
@@ -584,7 +584,7 @@ void sk_try(int index, uint32_t N, uint32_t K, const nfhip::Workspace& ws, SkPic
       if (kg > 1 && (tiles > (long)ws.cnt_len || (size_t)tiles * kg * (MT * 16 * G::kBN) > ws.part_floats)) break;
       const float t = sk_cost<QF, XT, MT, T, GN, NB, BUD>(SkJobs{1, {N}, {kg}}, K);
       const float key = t * (1.f + less * l2);
-      if (key < best.key) best = SkPick{key, t, index, GN * 16 + NB, kg};
+      if (key < best.key) best = SkPick{key, index, GN * 16 + NB, kg};
     }
   }
 }
@@ -676,34 +676,34 @@ SkPick sk_pick(uint32_t N, uint32_t K, const nfhip::Workspace& ws) {
 // picks' order.  An output depends on GN, NB and the K split (the order of
 // its sums) but not on T or the ring's depth, so a job gets the bits of its
 // own launch.  Declined (hipErrorNotSupported: the caller splits the group)
-// when the picks differ in order, or when one launch would take longer than
-// one each: K splits chosen for single launches can add up to a second round
-// of workgroups (Q8_0 f32 M = 64, two 14336x4096 jobs: 92 us as 448
-// workgroups of the single launches' variant, 41 us each alone).
+// only when the picks differ in order or the partial tiles do not fit: K
+// splits chosen for single launches can add up to further rounds of
+// workgroups, but one launch measured faster than one each all the same, us
+// apart / together: f32 M = 17, q, k and v of 8192, 1024 and 1024 rows at K =
+// 8192 Q4_0 36.7 / 34.8, Q8_0 41.4 / 39.0, two 14336x4096 44.5 / 43.0 and
+// 53.0 / 51.4; f16 M = 16, two 28672x8192 72.1 / 69.1 and 111.9 / 105.5; the
+// exception found, Q8_0 f16 M = 17, that q, k and v: 34.5 / 37.4.
 template <class QF, typename XT, int MT>
 hipError_t sk_group(const XT* A, const nfhip::GemvJob* jobs, uint32_t n, uint32_t M, uint32_t K,
                     const nfhip::Workspace& ws, hipStream_t s) {
   SkJobs js;
   js.n = n;
   SkPick pick;
-  float apart = 0.f;
   for (uint32_t j = 0; j < n; ++j) {
     const SkPick p = sk_pick<QF, XT, MT>(jobs[j].N, K, ws);
     if (p.variant < 0 || (j > 0 && p.order != pick.order)) return hipErrorNotSupported;
     js.N[j] = jobs[j].N;
     js.kg[j] = p.kg;
-    apart += p.cost;
     pick = p;
   }
   if (n > 1) {
-    pick.cost = 1e30f;
+    float best = 1e30f;
     sk_variants<MT>([&](auto i, auto t, auto gn, auto nb, auto bud) {
       if constexpr (SkGeom<QF, XT, MT, t(), gn(), nb(), bud()>::kOk) {
         const float c = sk_cost<QF, XT, MT, t(), gn(), nb(), bud()>(js, K);
-        if (gn() * 16 + nb() == pick.order && c < pick.cost) pick.cost = c, pick.variant = i();
+        if (gn() * 16 + nb() == pick.order && c < best) best = c, pick.variant = i();
       }
     });
-    if (pick.cost > apart) return hipErrorNotSupported;
   }
   hipError_t e = hipErrorNotSupported;
   sk_variants<MT>([&](auto i, auto t, auto gn, auto nb, auto bud) {

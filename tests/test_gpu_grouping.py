@@ -130,6 +130,29 @@ def test_run_tasks_merges_f16_batches(provider, oracle_mod, fmt, M, Ns, K):
         assert_close(c.astype(np.float32), ref.astype(np.float32), what=f"{fmt} {M}x{N}x{K}")
 
 
+# (format, f16, M, weight rows, K, launches): linears whose K splits add up to
+# more than one round of workgroups, one launch all the same; weights of more
+# than 16384 rows, whose sums run in another order, or of the f32 ring kernel
+# (Q4_0 above 8192 rows at M = 33..64), first in the list: alone, the rest
+# merged.
+@pytest.mark.parametrize("fmt,f16,M,Ns,K,launches", [
+    ("q4_0", False, 24, (8192, 1024, 1024), 8192, 1),
+    ("q8_0", False, 64, (2048, 300, 1100), 2048, 1),
+    ("q8_0", False, 40, (5632, 5632), 2048, 1),
+    ("q8_0", False, 64, (1024, 256, 256), 4096, 1),
+    ("q4_0", False, 24, (16400, 512, 640), 256, 2),
+    ("q8_0", False, 24, (16400, 512, 640), 256, 2),
+    ("q4_0", False, 48, (8200, 512, 640), 512, 2),
+    ("q4_0", False, 48, (8200, 16000), 512, 1),
+    ("q4_0", True, 12, (8192, 1024, 1024), 8192, 1),
+], ids=lambda v: str(v))
+def test_run_tasks_merges_uneven_linears(provider, fmt, f16, M, Ns, K, launches):
+    got, equal, _, _, out = _merged_and_apart(provider, fmt, f16, M, Ns, K, seed=M)
+    assert all(equal), equal
+    assert got == launches
+    assert all(np.isfinite(x).all() for x in out)
+
+
 def test_run_tasks_keeps_hazards_apart(provider, oracle_mod):
     """Two GEMVs over the same activations that write the same output are
     not merged; the output is the second one's, as in dispatch order."""
