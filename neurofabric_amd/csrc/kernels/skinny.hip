@@ -539,7 +539,7 @@ template <class QF, typename XT, int MT, int T, int GN, int NB, int BUD>
 float sk_cost(const SkJobs& jobs, uint32_t K) {
   typedef SkGeom<QF, XT, MT, T, GN, NB, BUD> G;
   constexpr SkCost c = SkCostOf<QF, XT>::k;
-  constexpr long per_cu = BUD > 79 ? 1 : 2, kCUs = 256;
+  constexpr long per_cu = BUD > 79 ? 1 : BUD > 53 ? 2 : 3, kCUs = 256;
   const int NC = (int)((K + G::kCK - 1) / G::kCK);
   long wgs = 0, split_wgs = 0, rows = 0;
   int chunks = 0, kg = 1;
@@ -627,10 +627,23 @@ hipError_t sk_launch(const XT* A, const nfhip::GemvJob* jobs, const int* kg, uin
   }
 }
 
+// Whether a variant is for rows of this K.  The 52 KB rings (two stages, three
+// workgroups per CU) are for weight rows of at most 768 bytes: such a row is
+// one to a few chunks, a deeper ring is never full, and what bounds a matrix
+// of many of them is the number of workgroups loading at once.  us at M = 8
+// with 78 KB rings -> with these: Q4_0 f32 128256x256 16.2 -> 12.0, 50257x768
+// 14.8 -> 13.2, f16 50257x768 12.9 -> 10.1, 128256x768 30.0 -> 24.8, Q8_0 f16
+// 65536x512 14.4 -> 12.9; past that the deeper rings win: Q8_0 f16 50257x1024
+// 18.2 against 19.6, f32 50257x768 16.3 against 17.1.
+template <class QF, int BUD>
+bool sk_suits(uint32_t K) {
+  return BUD > 53 || K / 32 * SkBlk<QF>::kBytes <= 768;
+}
+
 // The variants of each MT: f(std::integral_constant<int, T>, GN, NB, BUD).
-// One activation tile: two workgroups per CU (their rings fit half the LDS);
-// four and eight: one, and more waves along N, so that each activation
-// operand read from LDS feeds more weight tiles.
+// One activation tile: two or three workgroups per CU; four and eight: one,
+// and more waves along N, so that each activation operand read from LDS feeds
+// more weight tiles.
 template <int MT, class F>
 void sk_variants(F&& f) {
 #define SK_V(i, t, gn, nb, bud)                                                                              \
@@ -641,6 +654,8 @@ void sk_variants(F&& f) {
     SK_V(1, 2, 1, 1, 78);
     SK_V(2, 4, 1, 1, 78);
     SK_V(3, 2, 2, 1, 78);
+    SK_V(4, 4, 1, 1, 52);
+    SK_V(5, 4, 2, 1, 52);
   } else if constexpr (MT == 2) {
     SK_V(0, 1, 1, 1, 78);
     SK_V(1, 2, 1, 1, 78);
@@ -648,6 +663,7 @@ void sk_variants(F&& f) {
     SK_V(3, 4, 1, 1, 158);
     SK_V(4, 2, 2, 1, 78);
     SK_V(5, 4, 2, 1, 78);
+    SK_V(6, 4, 2, 1, 52);
   } else {
     SK_V(0, 1, 1, 1, 158);
     SK_V(1, 2, 1, 1, 158);
@@ -666,7 +682,8 @@ SkPick sk_pick(uint32_t N, uint32_t K, const nfhip::Workspace& ws) {
     // of a layer share a launch (Q8_0 M = 8, q, k and v of 4096, 1024 and
     // 1024 rows: 20.9 us when q alone took two waves along N); at 50257x768
     // M = 32 the two waves along N take 27.3 -> 19.2 us (Q4_0).
-    if (sizeof(XT) == 2 || gn() == (N > 16384 ? 2 : 1) || (N > 16384 && MT == 1)) sk_try<QF, XT, MT, t(), gn(), nb(), bud()>(i(), N, K, ws, best);
+    const bool order_ok = sizeof(XT) == 2 || gn() == (N > 16384 ? 2 : 1) || (N > 16384 && MT == 1);
+    if (order_ok && sk_suits<QF, bud()>(K)) sk_try<QF, XT, MT, t(), gn(), nb(), bud()>(i(), N, K, ws, best);
   });
   return best;
 }
@@ -701,7 +718,7 @@ hipError_t sk_group(const XT* A, const nfhip::GemvJob* jobs, uint32_t n, uint32_
     sk_variants<MT>([&](auto i, auto t, auto gn, auto nb, auto bud) {
       if constexpr (SkGeom<QF, XT, MT, t(), gn(), nb(), bud()>::kOk) {
         const float c = sk_cost<QF, XT, MT, t(), gn(), nb(), bud()>(js, K);
-        if (gn() * 16 + nb() == pick.order && c < best) best = c, pick.variant = i();
+        if (gn() * 16 + nb() == pick.order && sk_suits<QF, bud()>(K) && c < best) best = c, pick.variant = i();
       }
     });
   }

@@ -1,5 +1,5 @@
-// skinny_ring.hip — fused dequant + matmul of 33 to 64 f32 activation rows on
-// MFMA, weights streamed through an LDS ring.
+// skinny_ring.hip — fused dequant + matmul of up to 64 f32 activation rows on
+// MFMA, weights streamed through an LDS ring (33 rows and more, mostly).
 //
 // The same products as skinny.hip's f32 path (activations split into two
 // bf16 parts, exact bf16 codes, the block scale applied per block in fp32),
@@ -559,14 +559,22 @@ hipError_t ring_group_t(const float* A, const nfhip::GemvJob* jobs, uint32_t n, 
   }
 }
 
+template <class QF, int MT>
+hipError_t ring_mt(const float* A, const nfhip::GemvJob* jobs, uint32_t n, uint32_t M, uint32_t K,
+                   const nfhip::Workspace& ws, hipStream_t s) {
+  const int t = ring_t<QF, MT>(jobs[0].N);
+  if (t == 1) return ring_group_t<QF, MT, 1>(A, jobs, n, M, K, ws, s);
+  if (t == 2) return ring_group_t<QF, MT, 2>(A, jobs, n, M, K, ws, s);
+  if constexpr (MT == 4) return ring_group_t<QF, MT, 4>(A, jobs, n, M, K, ws, s);
+  return hipErrorNotSupported;  // ring_serves() sends no such weights here
+}
+
 template <class QF>
 hipError_t ring_dispatch(const float* A, const nfhip::GemvJob* jobs, uint32_t n, uint32_t M, uint32_t K,
                          const nfhip::Workspace& ws, hipStream_t s) {
-  switch (ring_t<QF, 4>(jobs[0].N)) {
-    case 1: return ring_group_t<QF, 4, 1>(A, jobs, n, M, K, ws, s);
-    case 2: return ring_group_t<QF, 4, 2>(A, jobs, n, M, K, ws, s);
-    default: return ring_group_t<QF, 4, 4>(A, jobs, n, M, K, ws, s);
-  }
+  if (M <= 16) return ring_mt<QF, 1>(A, jobs, n, M, K, ws, s);
+  if (M <= 32) return ring_mt<QF, 2>(A, jobs, n, M, K, ws, s);
+  return ring_mt<QF, 4>(A, jobs, n, M, K, ws, s);
 }
 
 }  // namespace ring
@@ -574,16 +582,21 @@ hipError_t ring_dispatch(const float* A, const nfhip::GemvJob* jobs, uint32_t n,
 
 namespace nfhip {
 
-// Where 33 to 64 f32 rows go to the ring kernel: two of its workgroups share
-// a CU, which pays once the other kernel's would need a second round.  f32,
-// M = 64, us in skinny.hip / here: Q4_0 50257x768 31.9 / 27.4, two 11008x4096
-// in a launch 69.9 / 63.0, but 4096x14336 35.6 / 40.9, 4096x4096 15.6 / 20.9;
-// Q8_0 14336x4096 43.9 / 40.8, q, k and v of 4096, 1024 and 1024 rows at
-// K = 4096 36.1 / 27.9, two 5632x2048 31.9 / 25.9, but 4096x1024 9.4 / 12.6,
-// 768x768 6.5 / 9.4.
+// Where f32 batches go to the ring kernel: two of its workgroups share a CU,
+// which pays once the other kernel's would need a second round.  us in
+// skinny.hip / here.  M = 64: Q4_0 50257x768 31.9 / 27.4, two 11008x4096 in a
+// launch 69.9 / 63.0, but 4096x14336 35.6 / 40.9, 4096x4096 15.6 / 20.9; Q8_0
+// 14336x4096 43.9 / 40.8, q, k and v of 4096, 1024 and 1024 rows at K = 4096
+// 36.1 / 27.9, two 5632x2048 31.9 / 25.9, 16384x256 10.6 / 9.1, but 4096x1024
+// 9.4 / 12.6, 768x768 6.5 / 9.4, 8192x256 6.3 / 9.7.  Up to 32 rows only where
+// a row is a single 256-element chunk of the other kernel, whose ring then
+// overlaps nothing: M = 8 Q8_0 24576x256 7.7 / 6.5, Q4_0 50257x256 9.4 / 7.7,
+// but 16384x256 5.8 / 6.2 and 5.0 / 5.5, 65536x256 10.2 / 13.9 and 9.6 / 11.0,
+// Q4_0 24576x512 7.4 / 7.7.
 bool ring_serves(QFmt q, EType t, uint32_t M, uint32_t N, uint32_t K) {
-  if (t != EType::F32 || M <= 32 || M > 64) return false;
-  return q == QFmt::Q4_0 ? N > 8192 : K > 2048 || (uint64_t)N * K > (4u << 20);
+  if (t != EType::F32 || M > 64) return false;
+  if (M <= 32) return K <= 256 && N > 16384 && N < 65536;
+  return N > 8192 || (q == QFmt::Q8_0 && (K > 2048 || (uint64_t)N * K > (4u << 20)));
 }
 
 hipError_t launch_skinny_ring(QFmt q, const void* A, const GemvJob* jobs, uint32_t n, uint32_t M, uint32_t K,

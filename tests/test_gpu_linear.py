@@ -194,6 +194,38 @@ def test_skinny_ring_f32_edges(provider, oracle_mod, fmt, shape):
 
 @pytest.mark.parametrize("fmt", ["q4_0", "q8_0"])
 @pytest.mark.parametrize("f16", [False, True], ids=["f32", "f16"])
+@pytest.mark.parametrize("M,N,K", [(3, 16400, 256), (16, 33001, 256), (17, 16385, 256), (32, 65535, 256),
+                                   (5, 65600, 256), (16, 50257, 512), (8, 24580, 768), (31, 65537, 512)])
+def test_short_weight_rows(provider, oracle_mod, fmt, f16, M, N, K):
+    """Tall matrices of short rows: the two-stage rings of three workgroups a
+    CU (f16 everywhere, f32 from 65536 rows or K = 512), whose ring is the
+    whole K or less, and for f32 K = 256 the ring kernel with one and two
+    activation tiles; ragged N.  First and last columns, twice in a row."""
+    old = provider.get_tuning()
+    dt, qdt = (abi.NF_DTYPE_F16 if f16 else abi.NF_DTYPE_F32), QDT[fmt]
+    npdt = np.float16 if f16 else np.float32
+    A, W = syn.activations(M, K, seed=M, dtype=npdt), syn.weights(fmt, N, K, seed=N)
+    a, w, c = provider.alloc_array(A, dt), provider.alloc_array(W, qdt), provider.alloc(dt, M * N * A.itemsize)
+    try:
+        _force_path(provider, "skinny", f16)
+        got = []
+        for _ in range(2):
+            provider.dispatch(f"dequant_{fmt}_linear" + ("_f16" if f16 else ""), [a, w], [c], M, N, K)
+            provider.synchronize()
+            got.append(c.download(npdt).reshape(M, N).copy())
+        assert np.array_equal(got[0].view(np.uint8), got[1].view(np.uint8))
+        for cols in ((0, 200), (N - 300, N)):
+            ref = oracle_mod.fused(A, W, fmt, M, N, K, f16=f16, cols=cols, threads=8)
+            ref = (ref.view(np.float16) if f16 else ref)[:, cols[0]:cols[1]].astype(np.float32)
+            assert_close(got[0][:, cols[0]:cols[1]].astype(np.float32), ref, what=f"{fmt} {M}x{N}x{K} {cols}")
+    finally:
+        provider.set_tuning(old)
+        for b in (a, w, c):
+            b.release()
+
+
+@pytest.mark.parametrize("fmt", ["q4_0", "q8_0"])
+@pytest.mark.parametrize("f16", [False, True], ids=["f32", "f16"])
 @pytest.mark.parametrize("shape", [(1, 1, 256), (7, 33, 1280), (16, 15, 768), (33, 513, 5376), (64, 129, 2304),
                                    (65, 150, 768), (128, 257, 1792)],
                          ids=lambda s: "x".join(map(str, s)))
