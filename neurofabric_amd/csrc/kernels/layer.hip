@@ -406,13 +406,22 @@ struct RopeJob {
   uint32_t rows_per_group, rows_per_pos;
 };
 
+// The first job's fields come first as plain scalars, so they are among the
+// arguments preloaded into SGPRs at wave launch and its workgroups load
+// nothing from the argument block: 2048 tokens of 32 heads x 128 13.5 -> 13.2
+// us in f32 and 11.7 -> 11.45 in f16, one token 3.52 -> 3.45.
 template <typename T>
-__global__ __launch_bounds__(kThreads) void rope_kernel(RopeJob<T> j0, RopeJob<T> j1, uint32_t wgs0,
-                                                        uint32_t head_dim, uint32_t step, float theta, bool batch) {
-  const bool second = blockIdx.x >= wgs0;
-  const RopeJob<T> job = second ? j1 : j0;
+__global__ __launch_bounds__(kThreads) void rope_kernel(const T* in0, T* out0, uint32_t head_dim, uint32_t rows_per_group0,
+                                                        uint32_t rows_per_pos0, uint32_t step, float theta, bool batch,
+                                                        uint32_t wgs0, uint64_t rows0, RopeJob<T> j1) {
+  RopeJob<T> job{in0, out0, rows0, rows_per_group0, rows_per_pos0};
+  uint32_t wg = blockIdx.x;
+  if (wg >= wgs0) {
+    job = j1;
+    wg -= wgs0;
+  }
   const uint32_t half = head_dim / 2;
-  const uint64_t id = (uint64_t)(blockIdx.x - (second ? wgs0 : 0)) * kThreads + threadIdx.x;
+  const uint64_t id = (uint64_t)wg * kThreads + threadIdx.x;
   const uint64_t grp = id / half;
   const uint32_t pair = (uint32_t)(id % half);
   const uint64_t r0 = grp * job.rows_per_group;
@@ -683,8 +692,9 @@ static hipError_t rope_jobs(bool batch, const RopeArgs* args, uint32_t njobs, ui
     wgs[i] = ((rows + per - 1) / per * (head_dim / 2) + kThreads - 1) / kThreads;
   }
   if (wgs[0] + wgs[1] == 0) return hipSuccess;
-  rope_kernel<T><<<dim3((unsigned)(wgs[0] + wgs[1])), kThreads, 0, s>>>(jobs[0], jobs[1], (uint32_t)wgs[0], head_dim,
-                                                                       step, theta, batch);
+  rope_kernel<T><<<dim3((unsigned)(wgs[0] + wgs[1])), kThreads, 0, s>>>(
+      jobs[0].in, jobs[0].out, head_dim, jobs[0].rows_per_group, jobs[0].rows_per_pos, step, theta, batch,
+      (uint32_t)wgs[0], jobs[0].rows, jobs[1]);
   return hipGetLastError();
 }
 

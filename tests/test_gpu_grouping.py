@@ -346,3 +346,34 @@ def test_run_tasks_layer_pairs(provider, pair, rows, dim, f16):
     finally:
         for b in bufs.values():
             b.release()
+
+
+@pytest.mark.parametrize("f16", [False, True], ids=["f32", "f16"])
+@pytest.mark.parametrize("tok,heads,D", [(1, (32, 8), 64), (5, (4, 12), 96), (130, (7, 1), 128), (700, (8, 2), 64)],
+                         ids=lambda v: str(v))
+def test_run_tasks_rope_pair_of_two_sizes(provider, tok, heads, D, f16):
+    """q and k of different head counts, the larger first or second, one
+    launch: the second job's workgroups begin where the first's end, and each
+    has its own group size.  The bits of one dispatch each."""
+    from neurofabric_amd.plugin import push_constants
+    npdt, dt = (np.float16, abi.NF_DTYPE_F16) if f16 else (np.float32, abi.NF_DTYPE_F32)
+    rng = np.random.default_rng(tok + D)
+    xs = [rng.standard_normal(tok * h * D).astype(npdt) for h in heads]
+    ins = [provider.alloc_array(x, dt) for x in xs]
+    outs = [provider.alloc(dt, x.nbytes) for x in xs]
+    tasks = [provider.task("rope_batch", [a], [o], pc=push_constants(seq_len=tok, n_heads=h, head_dim=D, theta=1e4,
+                                                                     step_idx=11)) for a, o, h in zip(ins, outs, heads)]
+    try:
+        before = provider.launch_count()
+        provider.run_tasks(_array(tasks), 1)
+        provider.synchronize()
+        assert provider.launch_count() - before == 1
+        got = [o.download(npdt).copy() for o in outs]
+        for td in tasks:
+            provider.check(provider.dispatch_task(td), "dispatch")
+        provider.synchronize()
+        for g, o in zip(got, outs):
+            assert np.array_equal(g.view(np.uint8), o.download(npdt).view(np.uint8))
+    finally:
+        for b in ins + outs:
+            b.release()
