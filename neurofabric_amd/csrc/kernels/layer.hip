@@ -71,11 +71,25 @@ __global__ __launch_bounds__(kThreads) void unary_kernel(const T* __restrict__ i
   }
 }
 
-// silu and the elementwise_mul of its output with `up`, both outputs written
-// (act may be gate or out; each element is read and written by one thread).
-// Bound by the launch at decode sizes, by HBM above: the second kernel's read
-// of act is saved.  5632 f32 elements: 2.4 + 2.3 us as two launches -> 2.5.
-template <typename T>
+// a * b with a as the instruction's first operand, which decides whose
+// payload a product of two NaNs has; the compiler may commute a plain product.
+__device__ __forceinline__ float mul_in_order(float a, float b) {
+  float r;
+  asm("v_mul_f32_e32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ half_t mul_in_order(half_t a, half_t b) {
+  half_t r;
+  asm("v_mul_f16_e32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+
+// silu and the elementwise_mul of its output with `up` (UP_FIRST: of `up`
+// with its output), both outputs written (act may be gate or out; each element
+// is read and written by one thread).  Bound by the launch at decode sizes, by
+// HBM above: the second kernel's read of act is saved.  5632 f32 elements:
+// 2.4 + 2.3 us as two launches -> 2.5.
+template <typename T, bool UP_FIRST>
 __global__ __launch_bounds__(kThreads) void silu_mul_kernel(const T* gate, const T* up, T* act, T* out, uint64_t n) {
   constexpr int V = 16 / (int)sizeof(T);
   typedef T vec_t __attribute__((ext_vector_type(V)));
@@ -84,15 +98,19 @@ __global__ __launch_bounds__(kThreads) void silu_mul_kernel(const T* gate, const
   if (i0 + V <= n) {
     vec_t x = *reinterpret_cast<const vec_t*>(gate + i0);
     const vec_t y = *reinterpret_cast<const vec_t*>(up + i0);
+    vec_t o;
 #pragma unroll
-    for (int j = 0; j < V; ++j) x[j] = (T)unary_f<EwFnK::Silu>((float)x[j]);
+    for (int j = 0; j < V; ++j) {
+      x[j] = (T)unary_f<EwFnK::Silu>((float)x[j]);
+      o[j] = UP_FIRST ? mul_in_order(y[j], x[j]) : mul_in_order(x[j], y[j]);
+    }
     *reinterpret_cast<vec_t*>(act + i0) = x;
-    *reinterpret_cast<vec_t*>(out + i0) = x * y;
+    *reinterpret_cast<vec_t*>(out + i0) = o;
   } else {
     for (uint64_t i = i0; i < n; ++i) {
       const T y = up[i], x = (T)unary_f<EwFnK::Silu>((float)gate[i]);
       act[i] = x;
-      out[i] = (T)(x * y);
+      out[i] = UP_FIRST ? mul_in_order(y, x) : mul_in_order(x, y);
     }
   }
 }
@@ -662,16 +680,22 @@ hipError_t launch_add_rms_norm(EType t, const void* a, const void* b, void* sum,
                          : rms_vec<float, true>(nc, a, b, sum, w, out, rows, dim, eps, s);
 }
 
-hipError_t launch_silu_mul(EType t, const void* gate, const void* up, void* act, void* out, uint64_t n, hipStream_t s) {
+template <typename T>
+static hipError_t silu_mul(const void* gate, const void* up, void* act, void* out, uint64_t n, bool up_first,
+                           hipStream_t s) {
+  using namespace nfk::layer;
+  constexpr uint64_t V = 16 / sizeof(T);
+  auto* kernel = up_first ? silu_mul_kernel<T, true> : silu_mul_kernel<T, false>;
+  kernel<<<grid_for((n + V - 1) / V), kThreads, 0, s>>>((const T*)gate, (const T*)up, (T*)act, (T*)out, n);
+  return hipGetLastError();
+}
+
+hipError_t launch_silu_mul(EType t, const void* gate, const void* up, void* act, void* out, uint64_t n, bool up_first,
+                           hipStream_t s) {
   using namespace nfk::layer;
   if (n == 0 || !a16(gate) || !a16(up) || !a16(act) || !a16(out)) return hipErrorNotSupported;
-  if (t == EType::F16)
-    silu_mul_kernel<half_t><<<grid_for((n + 7) / 8), kThreads, 0, s>>>((const half_t*)gate, (const half_t*)up,
-                                                                       (half_t*)act, (half_t*)out, n);
-  else
-    silu_mul_kernel<float><<<grid_for((n + 3) / 4), kThreads, 0, s>>>((const float*)gate, (const float*)up,
-                                                                      (float*)act, (float*)out, n);
-  return hipGetLastError();
+  return t == EType::F16 ? silu_mul<nfk::half_t>(gate, up, act, out, n, up_first, s)
+                         : silu_mul<float>(gate, up, act, out, n, up_first, s);
 }
 
 template <typename T>

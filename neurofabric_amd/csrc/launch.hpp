@@ -95,12 +95,14 @@ hipError_t launch_mock_prefill(const void* in, void* k, void* v, uint64_t nk, ui
 hipError_t launch_rms_norm(EType t, const void* in, const void* w, void* out, uint32_t rows, uint32_t dim, float eps,
                            hipStream_t s);
 // The residual addition and the norm after it: sum = a + b, out = rms_norm of
-// sum; and silu with the product after it: act = silu(gate), out = act * up.
+// sum; and silu with the product after it: act = silu(gate), out = act * up
+// (up_first: up * act, which differs in the payload where both are NaN).
 // The bits of the separate launches; hipErrorNotSupported for operands (odd
 // alignment, row lengths) that need them.
 hipError_t launch_add_rms_norm(EType t, const void* a, const void* b, void* sum, const void* w, void* out,
                                uint32_t rows, uint32_t dim, float eps, hipStream_t s);
-hipError_t launch_silu_mul(EType t, const void* gate, const void* up, void* act, void* out, uint64_t n, hipStream_t s);
+hipError_t launch_silu_mul(EType t, const void* gate, const void* up, void* act, void* out, uint64_t n, bool up_first,
+                           hipStream_t s);
 // batch: rope_batch ([seq, n_heads, head_dim], pos = token + step); else rope
 // (pos = step).  One or two jobs of n elements each in a launch.
 struct RopeArgs {

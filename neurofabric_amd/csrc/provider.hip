@@ -733,9 +733,9 @@ hipError_t run_group(const Prepared* prs, uint32_t n, const Workspace& ws, hipSt
       return launch_add_rms_norm(pl.c, prs[0].in[0]->dev, prs[0].in[1]->dev, prs[0].out[0]->dev, prs[1].in[1]->dev,
                                  prs[1].out[0]->dev, nx.lp.rows, nx.lp.dim, nx.lp.eps, s);
     case Path::Unary: {
-      const void* act = prs[0].out[0]->dev;
-      const void* up = prs[1].in[prs[1].in[0]->dev == act ? 1 : 0]->dev;
-      return launch_silu_mul(pl.c, prs[0].in[0]->dev, up, prs[0].out[0]->dev, prs[1].out[0]->dev, pl.count, s);
+      const bool up_first = prs[1].in[0]->dev != prs[0].out[0]->dev;
+      return launch_silu_mul(pl.c, prs[0].in[0]->dev, prs[1].in[up_first ? 0 : 1]->dev, prs[0].out[0]->dev,
+                             prs[1].out[0]->dev, pl.count, up_first, s);
     }
     default: return hipErrorNotSupported;
   }

@@ -377,3 +377,41 @@ def test_run_tasks_rope_pair_of_two_sizes(provider, tok, heads, D, f16):
     finally:
         for b in ins + outs:
             b.release()
+
+
+# Two NaNs of different payloads meet in the product and in the sum: the bits
+# of the fused launches are those of the separate ones for either operand order.
+@pytest.mark.parametrize("f16", [False, True], ids=["f32", "f16"])
+@pytest.mark.parametrize("pair", ["add_norm", "silu_mul", "silu_mul_swapped"])
+@pytest.mark.parametrize("dim", [64, 30])
+def test_run_tasks_layer_pairs_nan_payloads(provider, pair, dim, f16):
+    from neurofabric_amd.plugin import push_constants
+    if pair == "add_norm" and dim == 30:
+        pytest.skip("rows that are no whole number of chunks take two launches")
+    npdt, ut, dt = (np.float16, np.uint16, abi.NF_DTYPE_F16) if f16 else (np.float32, np.uint32, abi.NF_DTYPE_F32)
+    one = 0x7E01 if f16 else 0x7FC00001
+    data = {n: np.ones((3, dim), npdt) for n in "abust"}
+    for i, n in enumerate("abu"):
+        data[n].view(ut)[...] = one + np.arange(3 * dim, dtype=ut).reshape(3, dim) % 50 + 64 * i
+    for n in "bu":
+        data[n].view(ut)[1] |= 0x8000 if f16 else 0x80000000
+    data["w"] = np.ones(dim, np.float32)
+    bufs = {n: provider.alloc_array(x, abi.NF_DTYPE_F32 if n == "w" else dt) for n, x in data.items()}
+    steps, launches = FUSED[pair]
+    tasks = [provider.task(op, [bufs[n] for n in ins], [bufs[out]],
+                           pc=push_constants(seq_len=3, n_heads=1, head_dim=dim, epsilon=1e-5))
+             for op, ins, out in steps]
+    try:
+        before = provider.launch_count()
+        provider.run_tasks(_array(tasks), 1)
+        provider.synchronize()
+        assert provider.launch_count() - before == launches
+        got = {n: b.download(data[n].dtype).copy() for n, b in bufs.items()}
+        for td in tasks:
+            provider.check(provider.dispatch_task(td), "dispatch")
+        provider.synchronize()
+        for n, b in bufs.items():
+            assert np.array_equal(got[n].view(np.uint8), b.download(data[n].dtype).view(np.uint8)), n
+    finally:
+        for b in bufs.values():
+            b.release()
