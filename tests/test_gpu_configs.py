@@ -157,8 +157,8 @@ def test_config3_q8_0_ffn_and_lm_head(provider, oracle_mod, weights, M, NK):
 @pytest.mark.parametrize("NK", [(14336, 4096), (4096, 14336)], ids=["gate_up", "down"])
 def test_config3_forced_family(provider, oracle_mod, weights, path, M, NK):
     """The f32 families the switch points do not pick at these M: the
-    bf16-piece tiled GEMM at small batches, the small-batch kernel at M = 64
-    (two launches of 32 rows)."""
+    bf16-piece tiled GEMM at small batches; the small-batch kernel at M = 64
+    (one launch), pinned."""
     with forced(provider, path):
         kernel = planned_kernel(provider, "q8_0", M, *NK, False)
         want = {"skinny": "skinny_mfma_", "tiled": "gemm_mfma_"}[path]

@@ -130,6 +130,20 @@ def test_run_tasks_merges_f16_batches(provider, oracle_mod, fmt, M, Ns, K):
         assert_close(c.astype(np.float32), ref.astype(np.float32), what=f"{fmt} {M}x{N}x{K}")
 
 
+@pytest.mark.parametrize("fmt", ["q4_0", "q8_0"])
+@pytest.mark.parametrize("M", [24, 33, 64])
+@pytest.mark.parametrize("Ns,K", [((1024, 128, 128), 1024), ((2816, 2816), 1024), ((33, 700, 257, 1), 768)],
+                         ids=["gqa", "gate_up", "ragged"])
+def test_run_tasks_merges_f32_batches(provider, oracle_mod, fmt, M, Ns, K):
+    """f32 batches of two and four activation tiles off the ring kernel: one
+    launch, each linear with the K split, and the bits, of its own."""
+    launches, equal, A, Ws, out = _merged_and_apart(provider, fmt, False, M, Ns, K, seed=K)
+    assert all(equal), equal
+    assert launches == 1
+    for W, N, c in zip(Ws, Ns, out):
+        assert_close(c, oracle_mod.fused(A, W, fmt, M, N, K, threads=8), what=f"{fmt} {M}x{N}x{K}")
+
+
 # (format, f16, M, weight rows, K, launches): linears whose K splits add up to
 # more than one round of workgroups, one launch all the same; weights of more
 # than 16384 rows, whose sums run in another order, or of the f32 ring kernel
@@ -382,12 +396,10 @@ def test_run_tasks_rope_pair_of_two_sizes(provider, tok, heads, D, f16):
 # Two NaNs of different payloads meet in the product and in the sum: the bits
 # of the fused launches are those of the separate ones for either operand order.
 @pytest.mark.parametrize("f16", [False, True], ids=["f32", "f16"])
-@pytest.mark.parametrize("pair", ["add_norm", "silu_mul", "silu_mul_swapped"])
-@pytest.mark.parametrize("dim", [64, 30])
+@pytest.mark.parametrize("pair,dim", [("add_norm", 64), ("silu_mul", 64), ("silu_mul", 30), ("silu_mul_swapped", 64),
+                                      ("silu_mul_swapped", 30)])
 def test_run_tasks_layer_pairs_nan_payloads(provider, pair, dim, f16):
     from neurofabric_amd.plugin import push_constants
-    if pair == "add_norm" and dim == 30:
-        pytest.skip("rows that are no whole number of chunks take two launches")
     npdt, ut, dt = (np.float16, np.uint16, abi.NF_DTYPE_F16) if f16 else (np.float32, np.uint32, abi.NF_DTYPE_F32)
     one = 0x7E01 if f16 else 0x7FC00001
     data = {n: np.ones((3, dim), npdt) for n in "abust"}

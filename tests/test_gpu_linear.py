@@ -160,8 +160,8 @@ def test_small_f16_batches_on_the_tiled_kernels(provider, oracle_mod, fmt, M, N,
                          ids=lambda s: "x".join(map(str, s)))
 def test_skinny_mfma_shapes(provider, oracle_mod, fmt, f16, shape):
     """Small-batch MFMA kernel at ragged M/N, short and long K (the per-wave
-    K split and the LDS combine), rows beyond one launch (32 for f32, 64 for
-    f16); K % 256 != 0 falls back to the GEMV."""
+    K split and the LDS combine), rows beyond one launch (64 for f32, 128 for
+    f16); K % 256 != 0 falls back to the tiled GEMM or the GEMV."""
     M, N, K = shape
     old = provider.get_tuning()
     try:
@@ -176,12 +176,11 @@ def test_skinny_mfma_shapes(provider, oracle_mod, fmt, f16, shape):
                                    (33, 520, 1024), (64, 4096, 512), (48, 33000, 256), (64, 66000, 256)],
                          ids=lambda s: "x".join(map(str, s)))
 def test_skinny_ring_f32_edges(provider, oracle_mod, fmt, shape):
-    """The f32 small-batch kernel (weights through an LDS ring, activations
-    split once per workgroup): one, two and four 16-row activation tiles with
-    ragged M and N, a single chunk per workgroup and K split over
-    workgroups, and the 32- and 64-row waves of tall matrices (N >= 32768,
-    65536); up to 64 rows in one pass.  Each shape twice in a row (the
-    split-K arrival counters must be back at zero)."""
+    """f32 small batches: one, two and four 16-row activation tiles with ragged
+    M and N, a single chunk per workgroup and K split over workgroups, and
+    the ring kernel's 32- and 64-row waves of tall matrices (N >= 32768,
+    65536), unsplit; its other routes are in test_skinny_ring_routes.  Each
+    shape twice in a row (the split-K arrival counters must be back at zero)."""
     M, N, K = shape
     old = provider.get_tuning()
     try:
@@ -190,6 +189,26 @@ def test_skinny_ring_f32_edges(provider, oracle_mod, fmt, shape):
             check_fused(provider, oracle_mod, fmt, M, N, K, f16=False, seed=M * 5 + N + rep)
     finally:
         provider.set_tuning(old)
+
+
+@pytest.mark.parametrize("fmt,M,N,K", [
+    ("q4_0", 33, 8193, 1024), ("q4_0", 64, 8200, 2048), ("q4_0", 50, 14336, 512), ("q4_0", 64, 32769, 512),
+    ("q8_0", 64, 300, 4096), ("q8_0", 33, 129, 2304), ("q8_0", 47, 1, 4352), ("q8_0", 40, 2049, 2048),
+    ("q8_0", 64, 8193, 256), ("q8_0", 49, 33000, 512),
+], ids=lambda v: str(v))
+def test_skinny_ring_routes(provider, oracle_mod, fmt, M, N, K):
+    """What only the f32 ring kernel serves at 33 to 64 rows: 16-row waves just
+    above its limits and at ragged N, K in two halves (about 8200 and 14336
+    rows), up to sixteen parts (few rows) and undivided, 32-row waves, one
+    activation row past a 16-row tile and a full set.  The first and last
+    columns, twice in a row (the split-K counters must be back at zero)."""
+    A, W = syn.activations(M, K, seed=M), syn.weights(fmt, N, K, seed=N + K)
+    windows = [(0, N)] if N <= 600 else [(0, 200), (N - 300, N)]
+    refs = [oracle_mod.fused(A, W, fmt, M, N, K, cols=w, threads=8)[:, w[0]:w[1]] for w in windows]
+    for rep in range(2):
+        got = run_fused(provider, fmt, A, W, M, N, K, False)
+        for w, ref in zip(windows, refs):
+            assert_close(got[:, w[0]:w[1]], ref, what=f"{fmt} {M}x{N}x{K} {w} call {rep}")
 
 
 @pytest.mark.parametrize("fmt", ["q4_0", "q8_0"])
@@ -230,12 +249,13 @@ def test_short_weight_rows(provider, oracle_mod, fmt, f16, M, N, K):
                                    (65, 150, 768), (128, 257, 1792)],
                          ids=lambda s: "x".join(map(str, s)))
 def test_skinny_partial_chunks(provider, oracle_mod, fmt, f16, shape):
-    """Small-batch kernel where K is no multiple of its chunk (512 for f16
-    Q4_0, 256 or 128 else): the last chunk's loads past the row's end must
-    read zeros, not the next row.  One row and one column, ragged tiles, and
-    every count of 16-row activation tiles; twice in a row (split-K
-    counters).  The next row's blocks hold infinite scales in every second
-    row, so a byte of them in a finite row's sum shows."""
+    """Small-batch kernel at one row and one column, ragged tiles and every
+    count of 16-row activation tiles, twice in a row (split-K counters).  For
+    f16 Q4_0 the K values are also no multiple of the 512-element chunk of
+    waves side by side along K: the last chunk's loads past the row's end must
+    read zeros, not the next row, whose blocks hold infinite scales in every
+    second row, so a byte of them in a finite row's sum shows.  (Every other
+    chunk is 256 or 128 elements and divides K.)"""
     M, N, K = shape
     old = provider.get_tuning()
     W = syn.weights(fmt, N, K, seed=M + N).reshape(N, K // 32, -1).copy()
