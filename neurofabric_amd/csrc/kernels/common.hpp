@@ -162,4 +162,42 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
+// ---- rings of direct-to-LDS loads (skinny.hip, skinny_ring.hip) ---------------
+
+// Range-checked buffer resource (raw, no stride, `bytes` records).  A load
+// past them, or any load through a resource of zero bytes, returns zeros
+// without touching memory and still counts as an outstanding load, so a loop
+// can issue the same loads on every pass (its wait counts stay exact) while
+// those past its range cost nothing.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t sk_rsrc(const void* base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
+}
+
+// Buffer load to LDS, U = 16 or 4 bytes per lane: lane i writes lds + U*i from
+// offset voff (per lane) + soff (uniform).  (The builtin exists only in the
+// device pass.)
+template <int U>
+__device__ __forceinline__ void sk_dma(__amdgpu_buffer_rsrc_t r, void* lds, uint32_t voff, uint32_t soff = 0) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  auto* p = (__attribute__((address_space(3))) void*)lds;
+  if constexpr (U == 16)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, p, 16, (int)voff, (int)soff, 0, 0);
+  else
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, p, 4, (int)voff, (int)soff, 0, 0);
+#endif
+}
+
+// s_waitcnt immediate: vmcnt(v) (6 bits, split) and lgkmcnt(0), expcnt not waited on.
+constexpr int sk_wait_imm(int v) { return (v & 15) | ((v >> 4) << 14) | 0x0070; }
+
+// Workgroup barrier without a memory fence (the compiler's fence would wait
+// for every outstanding load, the ring's younger chunks included).
+__device__ __forceinline__ void sk_barrier() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 }  // namespace nfk

@@ -115,15 +115,15 @@ __device__ __forceinline__ bf16x8 sk_b_codes(const uint32_t (&q)[SkBlk<QF>::kSlo
 }
 
 // Geometry of a variant: MT 16-row activation tiles, T 16-row weight tiles
-// per wave, GN wave groups along N, NB units of K per wave and chunk, BUD KB
+// per wave, GN wave groups along N, a unit of K per wave and chunk, BUD KB
 // of LDS for the ring.
 constexpr int kSkWaves = 8;
-template <class QF, typename XT, int MT, int T, int GN, int NB, int BUD>
+template <class QF, typename XT, int MT, int T, int GN, int BUD>
 struct SkGeom {
   static constexpr int kGK = kSkWaves / GN;                 // waves splitting a chunk's K
   static constexpr int kBN = 16 * T * GN;                   // weight rows of a workgroup
   static constexpr int kUB = (sizeof(XT) == 2 && SkBlk<QF>::kSlot == 4) ? 2 : 1;  // blocks of a unit
-  static constexpr int kCK = 32 * kUB * kGK * NB;           // K of a chunk
+  static constexpr int kCK = 32 * kUB * kGK;           // K of a chunk
   static constexpr int kRB = kCK / 32 * SkBlk<QF>::kBytes;  // bytes of a weight row's chunk
   static constexpr int kUW = kRB % 16 == 0 ? 16 : 4;        // bytes per lane of a weight load
   static constexpr int kUR = kRB / kUW;                     // lane loads per row
@@ -148,38 +148,6 @@ struct SkGeom {
   static constexpr int kLds = kDump + 1024;
 };
 
-// Range-checked buffer resource (raw, no stride); with zero bytes every load
-// through it returns zeros and touches no memory.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t sk_rsrc(const void* base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
-}
-
-// Buffer load to LDS, U bytes per lane: lane i writes lds + U*i.  (The
-// builtin exists only in the device pass.)
-template <int U>
-__device__ __forceinline__ void sk_dma(__amdgpu_buffer_rsrc_t r, uint8_t* lds, uint32_t off) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  auto* p = (__attribute__((address_space(3))) void*)lds;
-  if constexpr (U == 16)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, p, 16, (int)off, 0, 0, 0);
-  else
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, p, 4, (int)off, 0, 0, 0);
-#endif
-}
-
-// s_waitcnt immediate: vmcnt(v) (6 bits, split) and lgkmcnt(0), expcnt not waited on.
-constexpr int sk_wait_imm(int v) { return (v & 15) | ((v >> 4) << 14) | 0x0070; }
-
-// Workgroup barrier without a memory fence (the compiler's fence would wait
-// for every outstanding load, the ring's younger chunks included).
-__device__ __forceinline__ void sk_barrier() {
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-}
-
 // Up to kSkGroupMax linears over the same activations in one launch: job j
 // owns workgroups begin[j] .. begin[j+1]-1: its row tiles, each split over
 // kg[j] consecutive workgroups along K, with arrival counters ctr[j] ..; a
@@ -199,13 +167,13 @@ struct SkGroup {
 // scalars (W0 = grp.W[0], ...), so they are among the arguments preloaded
 // into SGPRs at wave launch and a workgroup of job 0 (every workgroup of a
 // single launch) starts without a scalar load from the argument block.
-template <class QF, typename XT, int MT, int T, int GN, int NB, int BUD>
+template <class QF, typename XT, int MT, int T, int GN, int BUD>
 __global__ __launch_bounds__(64 * kSkWaves) void skinny_kernel(const XT* __restrict__ A,
                                                                const uint8_t* __restrict__ W0, int N0, int KG0, int b1,
                                                                int b2, int b3, int M, int K, void* C0, int CTR0,
                                                                float* __restrict__ ws_part,
                                                                uint32_t* __restrict__ ws_cnt, const SkGroup grp) {
-  typedef SkGeom<QF, XT, MT, T, GN, NB, BUD> G;
+  typedef SkGeom<QF, XT, MT, T, GN, BUD> G;
   constexpr bool kF32 = sizeof(XT) == 4;
   constexpr bool kQ4 = SkBlk<QF>::kSlot == 4;
   constexpr int S = G::kS, NT = 64 * kSkWaves;
@@ -304,15 +272,14 @@ __global__ __launch_bounds__(64 * kSkWaves) void skinny_kernel(const XT* __restr
     uint16_t d[T];
     u32x4 x[MT][XW];
   };
-  auto read_ops = [&](int st, int nb, Ops& o) {
+  auto read_ops = [&](int st, Ops& o) {
     const uint8_t* const xs = smem + st * G::kStage + G::kWB + r16 * (G::kXR * 16);
-    const int un = gk * NB + nb;  // unit of the chunk
     // first byte of the lane's block in its row's chunk, and of its codes, less the 2-byte misalignment
-    const int bo = kPair ? un * 36 + 18 * (s >> 1) : un * SkBlk<QF>::kBytes;
-    const int co = kPair ? bo + ((s >> 1) ? 2 : 0) + 8 * (s & 1) : bo + ((un & 1) ? 2 : 0) + SkBlk<QF>::kSlot * s;
+    const int bo = kPair ? gk * 36 + 18 * (s >> 1) : gk * SkBlk<QF>::kBytes;
+    const int co = kPair ? bo + ((s >> 1) ? 2 : 0) + 8 * (s & 1) : bo + ((gk & 1) ? 2 : 0) + SkBlk<QF>::kSlot * s;
     const uint8_t* const wr = smem + st * G::kStage + (gn * 16 * T + r16) * G::kRB;
     // element offsets of the lane's activations: two pieces of 8 (pair), of 4 (f32), or one of 8
-    const int e0 = kPair ? un * 64 + 32 * (s >> 1) + 8 * (s & 1) : un * 32 + (kQ4 ? 4 : 8) * s;
+    const int e0 = kPair ? gk * 64 + 32 * (s >> 1) + 8 * (s & 1) : gk * 32 + (kQ4 ? 4 : 8) * s;
     const int e1 = kPair || kQ4 ? e0 + 16 : e0 + 4;
     constexpr int EU = 16 / (int)sizeof(XT);
 #pragma unroll
@@ -329,9 +296,9 @@ __global__ __launch_bounds__(64 * kSkWaves) void skinny_kernel(const XT* __restr
       o.d[t] = *reinterpret_cast<const uint16_t*>(wr + 16 * t * G::kRB + bo);
     }
   };
-  auto compute = [&](int nb, const Ops& o) {
+  auto compute = [&](const Ops& o) {
     // bytes the codes sit into their first dword
-    const uint32_t sh = kPair ? ((s >> 1) ? 0u : 2u) : (((gk * NB + nb) & 1) ? 0u : 2u);
+    const uint32_t sh = kPair ? ((s >> 1) ? 0u : 2u) : ((gk & 1) ? 0u : 2u);
     if constexpr (kF32) {
       bf16x8 a1[MT], a2[MT];
       float4v b0[MT];
@@ -386,7 +353,7 @@ __global__ __launch_bounds__(64 * kSkWaves) void skinny_kernel(const XT* __restr
   };
   // Iteration i: wait for chunk i (the S-2 younger ones may stay in flight),
   // barrier (every wave's loads of chunk i are in, and every wave is done with
-  // chunk i-1, whose stage takes chunk i+S-1), read the first unit's operands,
+  // chunk i-1, whose stage takes chunk i+S-1), read the wave's operands,
   // issue chunk i+S-1, compute.
   const int nch = c_end - c_begin;
 #pragma unroll
@@ -396,16 +363,19 @@ __global__ __launch_bounds__(64 * kSkWaves) void skinny_kernel(const XT* __restr
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_waitcnt(sk_wait_imm((S - 2) * (G::kLW + G::kLX)));
     sk_barrier();
-    Ops o[2];
-    read_ops(st, 0, o[0]);
+    Ops o;
+    read_ops(st, o);
     __builtin_amdgcn_sched_barrier(0);
     issue(c_begin + i + S - 1, st == 0 ? S - 1 : st - 1);
     __builtin_amdgcn_sched_barrier(0);
+    // One unit a chunk.  As the body of a loop of one pass it is unrolled late,
+    // and the compiler orders the unpacking and the activation splits better:
+    // f32 Q8_0 M = 17 14336x4096 28.4 -> 26.5 us, f16 Q4_0 M = 32 50257x768
+    // 12.4 -> 11.6.
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-      if (nb + 1 < NB) read_ops(st, nb + 1, o[(nb + 1) & 1]);
+    for (int unit = 0; unit < 1; ++unit) {
       __builtin_amdgcn_sched_barrier(0);
-      compute(nb, o[nb & 1]);
+      compute(o);
       __builtin_amdgcn_sched_barrier(0);
     }
     st = st + 1 == S ? 0 : st + 1;
@@ -535,9 +505,9 @@ struct SkJobs {
   int kg[kSkGroupMax];
 };
 
-template <class QF, typename XT, int MT, int T, int GN, int NB, int BUD>
+template <class QF, typename XT, int MT, int T, int GN, int BUD>
 float sk_cost(const SkJobs& jobs, uint32_t K) {
-  typedef SkGeom<QF, XT, MT, T, GN, NB, BUD> G;
+  typedef SkGeom<QF, XT, MT, T, GN, BUD> G;
   constexpr SkCost c = SkCostOf<QF, XT>::k;
   constexpr long per_cu = BUD > 79 ? 1 : BUD > 53 ? 2 : 3, kCUs = 256;
   const int NC = (int)((K + G::kCK - 1) / G::kCK);
@@ -564,15 +534,15 @@ float sk_cost(const SkJobs& jobs, uint32_t K) {
 }
 
 // A launch's variant (index into sk_variants' list for its MT), the order of
-// its sums (GN and NB) and its K split.
+// its sums (GN) and its K split.
 struct SkPick {
   float key = 1e30f;
   int variant = -1, order = 0, kg = 1;
 };
 
-template <class QF, typename XT, int MT, int T, int GN, int NB, int BUD>
+template <class QF, typename XT, int MT, int T, int GN, int BUD>
 void sk_try(int index, uint32_t N, uint32_t K, const nfhip::Workspace& ws, SkPick& best) {
-  typedef SkGeom<QF, XT, MT, T, GN, NB, BUD> G;
+  typedef SkGeom<QF, XT, MT, T, GN, BUD> G;
   if constexpr (G::kOk) {
     const long tiles = ((long)N + G::kBN - 1) / G::kBN;
     const int NC = (int)((K + G::kCK - 1) / G::kCK);
@@ -582,19 +552,19 @@ void sk_try(int index, uint32_t N, uint32_t K, const nfhip::Workspace& ws, SkPic
     constexpr float less = MT <= 2 ? 0.06f : 0.f;
     for (int kg = 1, l2 = 0; kg <= 8 && kg <= NC; kg *= 2, ++l2) {
       if (kg > 1 && (tiles > (long)ws.cnt_len || (size_t)tiles * kg * (MT * 16 * G::kBN) > ws.part_floats)) break;
-      const float t = sk_cost<QF, XT, MT, T, GN, NB, BUD>(SkJobs{1, {N}, {kg}}, K);
+      const float t = sk_cost<QF, XT, MT, T, GN, BUD>(SkJobs{1, {N}, {kg}}, K);
       const float key = t * (1.f + less * l2);
-      if (key < best.key) best = SkPick{key, index, GN * 16 + NB, kg};
+      if (key < best.key) best = SkPick{key, index, GN, kg};
     }
   }
 }
 
-// One launch for n jobs (n = 1: a single linear) with variant <T, GN, NB,
-// BUD> and each job's own K split.
-template <class QF, typename XT, int MT, int T, int GN, int NB, int BUD>
+// One launch for n jobs (n = 1: a single linear) with variant <T, GN, BUD> and
+// each job's own K split.
+template <class QF, typename XT, int MT, int T, int GN, int BUD>
 hipError_t sk_launch(const XT* A, const nfhip::GemvJob* jobs, const int* kg, uint32_t n, uint32_t M, uint32_t K,
                      const nfhip::Workspace& ws, hipStream_t s) {
-  typedef SkGeom<QF, XT, MT, T, GN, NB, BUD> G;
+  typedef SkGeom<QF, XT, MT, T, GN, BUD> G;
   if constexpr (!G::kOk) {
     return hipErrorNotSupported;
   } else {
@@ -617,10 +587,10 @@ hipError_t sk_launch(const XT* A, const nfhip::GemvJob* jobs, const int* kg, uin
       return hipErrorNotSupported;
     for (int q = (int)n; q <= kSkGroupMax; ++q) grp.begin[q] = (int)wgs;
     static const hipError_t attr =
-        hipFuncSetAttribute(reinterpret_cast<const void*>(&skinny_kernel<QF, XT, MT, T, GN, NB, BUD>),
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&skinny_kernel<QF, XT, MT, T, GN, BUD>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, G::kLds);
     if (attr != hipSuccess) return attr;
-    skinny_kernel<QF, XT, MT, T, GN, NB, BUD><<<dim3((unsigned)wgs), dim3(64 * kSkWaves), G::kLds, s>>>(
+    skinny_kernel<QF, XT, MT, T, GN, BUD><<<dim3((unsigned)wgs), dim3(64 * kSkWaves), G::kLds, s>>>(
         A, grp.W[0], grp.N[0], grp.kg[0], grp.begin[1], grp.begin[2], grp.begin[3], (int)M, (int)K, grp.C[0],
         grp.ctr[0], ws.part, ws.cnt, grp);
     return hipGetLastError();
@@ -640,36 +610,36 @@ bool sk_suits(uint32_t K) {
   return BUD > 53 || K / 32 * SkBlk<QF>::kBytes <= 768;
 }
 
-// The variants of each MT: f(std::integral_constant<int, T>, GN, NB, BUD).
+// The variants of each MT: f(index, T, GN, BUD), integral constants.
 // One activation tile: two or three workgroups per CU; four and eight: one,
 // and more waves along N, so that each activation operand read from LDS feeds
 // more weight tiles.
 template <int MT, class F>
 void sk_variants(F&& f) {
-#define SK_V(i, t, gn, nb, bud)                                                                              \
+#define SK_V(i, t, gn, bud)                                                                                \
   f(std::integral_constant<int, i>{}, std::integral_constant<int, t>{}, std::integral_constant<int, gn>{}, \
-    std::integral_constant<int, nb>{}, std::integral_constant<int, bud>{})
+    std::integral_constant<int, bud>{})
   if constexpr (MT == 1) {
-    SK_V(0, 1, 1, 1, 78);
-    SK_V(1, 2, 1, 1, 78);
-    SK_V(2, 4, 1, 1, 78);
-    SK_V(3, 2, 2, 1, 78);
-    SK_V(4, 4, 1, 1, 52);
-    SK_V(5, 4, 2, 1, 52);
+    SK_V(0, 1, 1, 78);
+    SK_V(1, 2, 1, 78);
+    SK_V(2, 4, 1, 78);
+    SK_V(3, 2, 2, 78);
+    SK_V(4, 4, 1, 52);
+    SK_V(5, 4, 2, 52);
   } else if constexpr (MT == 2) {
-    SK_V(0, 1, 1, 1, 78);
-    SK_V(1, 2, 1, 1, 78);
-    SK_V(2, 2, 1, 1, 158);
-    SK_V(3, 4, 1, 1, 158);
-    SK_V(4, 2, 2, 1, 78);
-    SK_V(5, 4, 2, 1, 78);
-    SK_V(6, 4, 2, 1, 52);
+    SK_V(0, 1, 1, 78);
+    SK_V(1, 2, 1, 78);
+    SK_V(2, 2, 1, 158);
+    SK_V(3, 4, 1, 158);
+    SK_V(4, 2, 2, 78);
+    SK_V(5, 4, 2, 78);
+    SK_V(6, 4, 2, 52);
   } else {
-    SK_V(0, 1, 1, 1, 158);
-    SK_V(1, 2, 1, 1, 158);
-    SK_V(2, 4, 1, 1, 158);
-    SK_V(3, 2, 2, 1, 158);
-    SK_V(4, 4, 2, 1, 158);
+    SK_V(0, 1, 1, 158);
+    SK_V(1, 2, 1, 158);
+    SK_V(2, 4, 1, 158);
+    SK_V(3, 2, 2, 158);
+    SK_V(4, 4, 2, 158);
   }
 #undef SK_V
 }
@@ -677,20 +647,20 @@ void sk_variants(F&& f) {
 template <class QF, typename XT, int MT>
 SkPick sk_pick(uint32_t N, uint32_t K, const nfhip::Workspace& ws) {
   SkPick best;
-  sk_variants<MT>([&](auto i, auto t, auto gn, auto nb, auto bud) {
+  sk_variants<MT>([&](auto i, auto t, auto gn, auto bud) {
     // f32: one order of sums for all but the tallest weights, so the linears
     // of a layer share a launch (Q8_0 M = 8, q, k and v of 4096, 1024 and
     // 1024 rows: 20.9 us when q alone took two waves along N); at 50257x768
     // M = 32 the two waves along N take 27.3 -> 19.2 us (Q4_0).
     const bool order_ok = sizeof(XT) == 2 || gn() == (N > 16384 ? 2 : 1) || (N > 16384 && MT == 1);
-    if (order_ok && sk_suits<QF, bud()>(K)) sk_try<QF, XT, MT, t(), gn(), nb(), bud()>(i(), N, K, ws, best);
+    if (order_ok && sk_suits<QF, bud()>(K)) sk_try<QF, XT, MT, t(), gn(), bud()>(i(), N, K, ws, best);
   });
   return best;
 }
 
 // A group of jobs: each with the K split of its own pick, all with the
 // variant the cost model finds fastest for the whole among those of the
-// picks' order.  An output depends on GN, NB and the K split (the order of
+// picks' order.  An output depends on GN and the K split (the order of
 // its sums) but not on T or the ring's depth, so a job gets the bits of its
 // own launch.  Declined (hipErrorNotSupported: the caller splits the group)
 // only when the picks differ in order or the partial tiles do not fit: K
@@ -715,16 +685,16 @@ hipError_t sk_group(const XT* A, const nfhip::GemvJob* jobs, uint32_t n, uint32_
   }
   if (n > 1) {
     float best = 1e30f;
-    sk_variants<MT>([&](auto i, auto t, auto gn, auto nb, auto bud) {
-      if constexpr (SkGeom<QF, XT, MT, t(), gn(), nb(), bud()>::kOk) {
-        const float c = sk_cost<QF, XT, MT, t(), gn(), nb(), bud()>(js, K);
-        if (gn() * 16 + nb() == pick.order && sk_suits<QF, bud()>(K) && c < best) best = c, pick.variant = i();
+    sk_variants<MT>([&](auto i, auto t, auto gn, auto bud) {
+      if constexpr (SkGeom<QF, XT, MT, t(), gn(), bud()>::kOk) {
+        const float c = sk_cost<QF, XT, MT, t(), gn(), bud()>(js, K);
+        if (gn() == pick.order && sk_suits<QF, bud()>(K) && c < best) best = c, pick.variant = i();
       }
     });
   }
   hipError_t e = hipErrorNotSupported;
-  sk_variants<MT>([&](auto i, auto t, auto gn, auto nb, auto bud) {
-    if (i() == pick.variant) e = sk_launch<QF, XT, MT, t(), gn(), nb(), bud()>(A, jobs, js.kg, n, M, K, ws, s);
+  sk_variants<MT>([&](auto i, auto t, auto gn, auto bud) {
+    if (i() == pick.variant) e = sk_launch<QF, XT, MT, t(), gn(), bud()>(A, jobs, js.kg, n, M, K, ws, s);
   });
   return e;
 }

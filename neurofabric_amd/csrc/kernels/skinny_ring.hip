@@ -6,10 +6,11 @@
 // split for weights with many rows: every wave of a workgroup owns weight
 // rows and walks the workgroup's whole K range, in chunks of 64 elements, so
 // the workgroup needs 32 KB of split activations and a small weight ring and
-// two fit on a CU; skinny.hip's workgroups (whole 256-element activation
-// chunks in the ring) fill one.  Bound by the fp32 scale FMAs and unpacking
-// beside the MFMAs.  ring_serves() has the line between the two, with both
-// sides' times.
+// two fit on a CU (with one or two 16-row tiles a wave; from 65536 rows on,
+// with four, one); skinny.hip's workgroups for these batches (whole
+// 256-element activation chunks in the ring) fill one.  Bound by the fp32
+// scale FMAs and unpacking beside the MFMAs.  ring_serves() has the line
+// between the two, with both sides' times.
 //
 // MFMA v_mfma_f32_16x16x32 (bf16): A = activations (16 rows of M), B =
 // weights (16 rows of N), D[m][n] = sum over 32 k.  Lane l:
@@ -34,26 +35,6 @@ template <> struct SkW<Q4_0> {
 template <> struct SkW<Q8_0> {
   static constexpr int kPairBytes = 68, kLoads = 7;
 };
-
-// The dwords of pair `p` of weight row `row` that slot s needs.
-template <class QF>
-__device__ __forceinline__ void sk_load_w(const uint32_t* __restrict__ pr, int s, uint32_t (&w)[SkW<QF>::kLoads]) {
-  if constexpr (SkW<QF>::kLoads == 5) {
-    w[0] = pr[s];      // block 0 codes, realigned with w[1]
-    w[1] = pr[s + 1];
-    w[2] = pr[5 + s];  // block 1 codes
-    w[3] = pr[0];      // block 0 scale (low half)
-    w[4] = pr[4];      // block 1 scale (high half)
-  } else {
-    w[0] = pr[2 * s];  // block 0 codes: bytes 2+8s .. 9+8s across three dwords
-    w[1] = pr[2 * s + 1];
-    w[2] = pr[2 * s + 2];
-    w[3] = pr[9 + 2 * s];   // block 1 codes
-    w[4] = pr[10 + 2 * s];
-    w[5] = pr[0];      // block 0 scale (low half)
-    w[6] = pr[8];      // block 1 scale (high half)
-  }
-}
 
 template <class QF>
 __device__ __forceinline__ uint32_t sk_scale_bits(const uint32_t (&w)[SkW<QF>::kLoads], int h) {
@@ -84,16 +65,6 @@ __device__ __forceinline__ bf16x8 sk_b_codes(const uint32_t (&w)[SkW<QF>::kLoads
   return __builtin_bit_cast(bf16x8, o);
 }
 
-// Range-checked buffer loads (gfx9 raw buffer resource: base, no stride,
-// num_records bytes).  A load through a resource with num_records = 0
-// returns zeros without touching memory and still counts as an outstanding
-// load, which lets a loop issue the same loads on every pass (so the
-// compiler's wait counts stay exact) while loads past a wave's range cost
-// nothing.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t sk_rsrc(const void* base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
-}
-
 constexpr int kSkGroupMax = nfhip::kGemvGroupMax;
 static_assert(kSkGroupMax == 4, "the kernel passes begin[1..3] as scalar arguments");
 
@@ -111,7 +82,7 @@ __device__ __forceinline__ int group_job(int b1, int b2, int b3) {
 
 // A workgroup is 8 waves (two per SIMD) over 128*T weight rows (wave w: rows
 // 16T*w .. 16T*w + 16T-1 as T 16-row tiles), and all waves walk the same K
-// range chunk by chunk; a chunk is CHP pairs (64*CHP elements).  The weight
+// range chunk by chunk; a chunk is a pair of blocks (64 elements).  The weight
 // ring has S stages; chunk i+S-1 is requested while chunk i is computed, by
 // buffer_load ... lds, which writes LDS without passing through registers
 // (so S-1 chunks in flight cost no registers), range-checked: chunks past
@@ -125,18 +96,18 @@ __device__ __forceinline__ int group_job(int b1, int b2, int b3) {
 // chunk i splits them once for the whole workgroup into the two bf16 pieces
 // of the MFMA operand (x ~ b1 + b2, split2), stored in operand order in one
 // of two LDS buffers, so a wave reads each piece with one conflict-free
-// ds_read_b128.  Every wave then runs the MFMA chain on its tiles (exact bf16 codes, two chained MFMAs, the block scale applied per
-// block in fp32).
+// ds_read_b128.  Every wave then runs the MFMA chain on its tiles (exact bf16
+// codes, two chained MFMAs, the block scale applied per block in fp32).
 //
-// With K split over KG workgroups (grid y), each parks its partial tile and
+// With K split over KG workgroups, each parks its partial tile and
 // the last to arrive adds the KG tiles in order kg = 0..KG-1 (deterministic)
 // and stores C.
-template <class QF, int MT, int T, int CHP>
+template <class QF, int MT, int T>
 struct RingGeom {
   static constexpr int kWaves = 8;
   static constexpr int kPB = SkW<QF>::kPairBytes, kPD = kPB / 4;
   static constexpr int kRW = 16 * T;                   // weight rows per wave
-  static constexpr int kWRow = CHP * kPD;              // dwords per staged weight row
+  static constexpr int kWRow = kPD;                    // dwords per staged weight row
   static constexpr int kWDw = kRW * kWRow;             // weight dwords of a wave per chunk
   static constexpr int kJW = (kWDw + 63) / 64;         // dword loads per lane per chunk
   // A wave's area in a stage is padded to whole loads: every lane issues all
@@ -145,32 +116,10 @@ struct RingGeom {
   // wait analysis drop count and wait for loads issued an iteration later.
   static constexpr int kWArea = kJW * 64;
   static constexpr int kStage = kWaves * kWArea;       // dwords of a stage
-  static constexpr int kUnits = CHP * 2 * MT * 64;     // A operands (lane slots) per chunk
+  static constexpr int kUnits = 2 * MT * 64;           // A operands (lane slots) per chunk
   static constexpr int kUPT = (kUnits + 511) / 512;    // A operands per thread
   static constexpr int kXB = kUnits * 8;               // dwords of one split buffer (two bf16x8 each)
 };
-
-// s_waitcnt immediate: vmcnt(v) (6 bits, split), expcnt and lgkmcnt not waited on.
-constexpr int sk_vmcnt_imm(int v) { return (v & 15) | ((v >> 4) << 14) | 0x0070 | 0x0F00; }
-
-// Buffer load to LDS: lane i writes lds + 4*i; the builtin exists only in
-// the device pass.
-__device__ __forceinline__ void sk_dma4(__amdgpu_buffer_rsrc_t r, uint32_t* lds, uint32_t voff, uint32_t soff) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 4, (int)voff,
-                                           (int)soff, 0, 0);
-#endif
-}
-
-// Workgroup barrier without a memory fence (the compiler's fence would wait
-// for every outstanding load, including the ring's younger chunks).
-__device__ __forceinline__ void sk_barrier() {
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-}
 
 // Jobs of one ring launch: job j owns workgroups begin[j] .. begin[j+1]-1,
 // tiles[j] row tiles with its own K split kg[j] (tile-major: the kg[j]
@@ -191,7 +140,7 @@ constexpr int kRingGatherF4 = 16;
 
 // Arguments: job 0's fields first (W0 = grp.W[0], N0,
 // KG0 = grp.kg[0], C0, CTR0 = grp.ctr[0]).
-template <class QF, int MT, int T, int CHP, int S>
+template <class QF, int MT, int T, int S>
 __global__ __launch_bounds__(512) void skinny_ring_kernel(const float* __restrict__ A,
                                                          const uint8_t* __restrict__ W0, int N0, int KG0, int b1,
                                                          int b2, int b3, int M, int K, void* C0, int CTR0,
@@ -211,7 +160,7 @@ __global__ __launch_bounds__(512) void skinny_ring_kernel(const float* __restric
   }
   float* __restrict__ C = static_cast<float*>(Cv);
   const int local = (int)blockIdx.x - wg0, tile = local / KG, kg = local - tile * KG;
-  typedef RingGeom<QF, MT, T, CHP> G;
+  typedef RingGeom<QF, MT, T> G;
   constexpr bool kQ4 = SkW<QF>::kLoads == 5;
   constexpr int WL = SkW<QF>::kLoads;
   constexpr int RW = G::kRW, NW = G::kWaves, UPT = G::kUPT;
@@ -222,7 +171,7 @@ __global__ __launch_bounds__(512) void skinny_ring_kernel(const float* __restric
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, s = lane >> 4;
-  const int NC = (K >> 6) / CHP;
+  const int NC = K >> 6;
   const int n0 = tile * (NW * RW) + wave * RW;  // this wave's first row
   const int c_begin = (int)((long)NC * kg / KG), c_end = (int)((long)NC * (kg + 1) / KG);
 
@@ -242,16 +191,16 @@ __global__ __launch_bounds__(512) void skinny_ring_kernel(const float* __restric
   auto fetch_w = [&](int c, int st) {
     const bool live = c < c_end;
     const __amdgpu_buffer_rsrc_t rw = sk_rsrc(W, __builtin_amdgcn_readfirstlane(live ? w_bytes : 0u));
-    const uint32_t wo = __builtin_amdgcn_readfirstlane(live ? (uint32_t)c * (uint32_t)(CHP * G::kPB) : 0u);
+    const uint32_t wo = __builtin_amdgcn_readfirstlane(live ? (uint32_t)c * (uint32_t)G::kPB : 0u);
     uint32_t* wsb = smem + st * G::kStage + wave * G::kWArea;
 #pragma unroll
-    for (int j = 0; j < G::kJW; ++j) sk_dma4(rw, wsb + 64 * j, wsrc[j], wo);
+    for (int j = 0; j < G::kJW; ++j) sk_dma<4>(rw, wsb + 64 * j, wsrc[j], wo);
   };
 
-  // A operands: unit u = ((pi * 2 + h) * MT + mt) * 64 + l is the operand of
-  // lane l (row 16mt + l%16, slot l/16) for block h of pair pi of a chunk:
-  // activations k = 64pi + 32h + {off0 .. off0+3, off1 .. off1+3} of its row
-  // (the k order of the lane's weight codes).  Thread tid takes units tid,
+  // A operands: unit u = (h * MT + mt) * 64 + l is the operand of lane l (row
+  // 16mt + l%16, slot l/16) for block h of a chunk: activations k = 32h +
+  // {off0 .. off0+3, off1 .. off1+3} of its row (the k order of the lane's
+  // weight codes).  Thread tid takes units tid,
   // tid + 512, ...; piece k (0: hi, 1: lo) of unit u goes to 16-byte slot
   // ((u / 64) * 2 + k) * 64 + l of a split buffer, so a wave's read of one
   // piece covers 1 KB contiguously.
@@ -262,10 +211,10 @@ __global__ __launch_bounds__(512) void skinny_ring_kernel(const float* __restric
     const int u = tid + 512 * k;
     xlive[k] = G::kUnits % 512 == 0 || u < G::kUnits;
     const int uu = xlive[k] ? u : 0;
-    const int l = uu & 63, mt = (uu >> 6) % MT, ph = (uu >> 6) / MT, h = ph & 1, pi = ph >> 1;
+    const int l = uu & 63, mt = (uu >> 6) % MT, h = (uu >> 6) / MT;
     const int m = 16 * mt + (l & 15);
     const int mm = m < M ? m : M - 1;
-    xoff[k] = ((uint32_t)mm * (uint32_t)K + (uint32_t)(64 * pi + 32 * h + (kQ4 ? 4 : 8) * (l >> 4))) * 4u;
+    xoff[k] = ((uint32_t)mm * (uint32_t)K + (uint32_t)(32 * h + (kQ4 ? 4 : 8) * (l >> 4))) * 4u;
   }
   const uint32_t x_bytes = (uint32_t)M * (uint32_t)K * 4u;
   typedef float4v XSet[UPT][2];
@@ -273,7 +222,7 @@ __global__ __launch_bounds__(512) void skinny_ring_kernel(const float* __restric
   auto load_x = [&](int c, XSet& x) {
     const bool live = c < c_end;
     const __amdgpu_buffer_rsrc_t rx = sk_rsrc(A, __builtin_amdgcn_readfirstlane(live ? x_bytes : 0u));
-    const uint32_t xo = __builtin_amdgcn_readfirstlane(live ? (uint32_t)c * (CHP * 256u) : 0u);
+    const uint32_t xo = __builtin_amdgcn_readfirstlane(live ? (uint32_t)c * 256u : 0u);
 #pragma unroll
     for (int k = 0; k < UPT; ++k) {
       x[k][0] = __builtin_bit_cast(float4v, __builtin_amdgcn_raw_buffer_load_b128(rx, xoff[k], xo, 0));
@@ -309,49 +258,56 @@ __global__ __launch_bounds__(512) void skinny_ring_kernel(const float* __restric
   auto compute = [&](int st, const uint32_t* xb) {
     const uint32_t* wsb = smem + st * G::kStage + wave * G::kWArea;
 #pragma unroll
-    for (int pi = 0; pi < CHP; ++pi)
+    for (int h = 0; h < 2; ++h) {
+      bf16x8 a1[MT], a2[MT];
+      float4v base[MT];
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        bf16x8 a1[MT], a2[MT];
-        float4v base[MT];
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-          const uint32_t* up = xb + ((((pi * 2 + h) * MT + mt) * 2) * 64 + lane) * 4;
-          a1[mt] = *reinterpret_cast<const bf16x8*>(up);
-          a2[mt] = *reinterpret_cast<const bf16x8*>(up + 256);
-          base[mt] = float4v{0.f, 0.f, 0.f, 0.f};
-          if constexpr (kQ4) {
-            // sum_k (-136) * x, the offset of the 128 + n codes, shared by
-            // all weight tiles
-            const __bf16 c8 = (__bf16)(-136.0f);
-            const bf16x8 bc = {c8, c8, c8, c8, c8, c8, c8, c8};
-            base[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[mt], bc, base[mt], 0, 0, 0);
-            base[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2[mt], bc, base[mt], 0, 0, 0);
-          }
-        }
-#pragma unroll
-        for (int t = 0; t < T; ++t) {
-          const uint32_t* pr = wsb + (16 * t + r16) * G::kWRow + pi * G::kPD;
-          uint32_t w[WL];
-          if constexpr (WL == 5) {
-            w[0] = pr[s]; w[1] = pr[s + 1]; w[2] = pr[5 + s]; w[3] = pr[0]; w[4] = pr[4];
-          } else {
-            w[0] = pr[2 * s]; w[1] = pr[2 * s + 1]; w[2] = pr[2 * s + 2];
-            w[3] = pr[9 + 2 * s]; w[4] = pr[10 + 2 * s]; w[5] = pr[0]; w[6] = pr[8];
-          }
-          const bf16x8 b = sk_b_codes<QF>(w, h);
-          float d = h2f_bits((uint16_t)sk_scale_bits<QF>(w, h));
-          if (!wvalid[t]) d = 0.f;
-#pragma unroll
-          for (int mt = 0; mt < MT; ++mt) {
-            float4v dd = base[mt];
-            dd = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[mt], b, dd, 0, 0, 0);
-            dd = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2[mt], b, dd, 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) acc[mt][t][i] = __builtin_fmaf(d, dd[i], acc[mt][t][i]);
-          }
+      for (int mt = 0; mt < MT; ++mt) {
+        const uint32_t* up = xb + (((h * MT + mt) * 2) * 64 + lane) * 4;
+        a1[mt] = *reinterpret_cast<const bf16x8*>(up);
+        a2[mt] = *reinterpret_cast<const bf16x8*>(up + 256);
+        base[mt] = float4v{0.f, 0.f, 0.f, 0.f};
+        if constexpr (kQ4) {
+          // sum_k (-136) * x, the offset of the 128 + n codes, shared by
+          // all weight tiles
+          const __bf16 c8 = (__bf16)(-136.0f);
+          const bf16x8 bc = {c8, c8, c8, c8, c8, c8, c8, c8};
+          base[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[mt], bc, base[mt], 0, 0, 0);
+          base[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2[mt], bc, base[mt], 0, 0, 0);
         }
       }
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        const uint32_t* pr = wsb + (16 * t + r16) * G::kWRow;
+        uint32_t w[WL];
+        if constexpr (WL == 5) {
+          w[0] = pr[s];      // block 0 codes, realigned with w[1]
+          w[1] = pr[s + 1];
+          w[2] = pr[5 + s];  // block 1 codes
+          w[3] = pr[0];      // block 0 scale (low half)
+          w[4] = pr[4];      // block 1 scale (high half)
+        } else {
+          w[0] = pr[2 * s];  // block 0 codes: bytes 2+8s .. 9+8s across three dwords
+          w[1] = pr[2 * s + 1];
+          w[2] = pr[2 * s + 2];
+          w[3] = pr[9 + 2 * s];  // block 1 codes
+          w[4] = pr[10 + 2 * s];
+          w[5] = pr[0];      // block 0 scale (low half)
+          w[6] = pr[8];      // block 1 scale (high half)
+        }
+        const bf16x8 b = sk_b_codes<QF>(w, h);
+        float d = h2f_bits((uint16_t)sk_scale_bits<QF>(w, h));
+        if (!wvalid[t]) d = 0.f;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+          float4v dd = base[mt];
+          dd = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[mt], b, dd, 0, 0, 0);
+          dd = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2[mt], b, dd, 0, 0, 0);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[mt][t][i] = __builtin_fmaf(d, dd[i], acc[mt][t][i]);
+        }
+      }
+    }
   };
 
   // Pipeline.  Before the loop: chunk 0's activations, the weights of
@@ -390,7 +346,7 @@ __global__ __launch_bounds__(512) void skinny_ring_kernel(const float* __restric
   auto iteration = [&](auto pc, int i) {
     constexpr int p = decltype(pc)::value;
     __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_waitcnt(sk_vmcnt_imm((S - 2) * G::kJW + 2 * UPT) & ~0x0F00);
+    __builtin_amdgcn_s_waitcnt(sk_wait_imm((S - 2) * G::kJW + 2 * UPT));
     sk_barrier();
     load_x(c_begin + i + 2, xr[p]);
     __builtin_amdgcn_sched_barrier(0);
@@ -481,7 +437,7 @@ __global__ __launch_bounds__(512) void skinny_ring_kernel(const float* __restric
 // fit in 160 KB of LDS beside the two split buffers, at most 4, at least 3.
 template <class QF, int MT, int T>
 struct RingCfg {
-  typedef RingGeom<QF, MT, T, 1> G;
+  typedef RingGeom<QF, MT, T> G;
   static constexpr int kFree = 160 * 1024 / 4 - 2 * G::kXB - 64;  // dwords (64 for the static LDS)
   static constexpr int kSLds = kFree / G::kStage, kSVm = 2 + (63 - 2 * G::kUPT) / G::kJW;  // LDS, vmcnt field
   static constexpr int kSMax = 4;  // deeper rings measured slower (fewer workgroups per CU)
@@ -549,10 +505,10 @@ hipError_t ring_group_t(const float* A, const nfhip::GemvJob* jobs, uint32_t n, 
       return hipErrorNotSupported;
     for (int q = (int)n; q <= kSkGroupMax; ++q) grp.begin[q] = (int)wgs;
     static const hipError_t attr =
-        hipFuncSetAttribute(reinterpret_cast<const void*>(&skinny_ring_kernel<QF, MT, T, 1, Cfg::kS>),
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&skinny_ring_kernel<QF, MT, T, Cfg::kS>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::kLds);
     if (attr != hipSuccess) return attr;
-    skinny_ring_kernel<QF, MT, T, 1, Cfg::kS><<<dim3((unsigned)wgs), dim3(512), Cfg::kLds, s>>>(
+    skinny_ring_kernel<QF, MT, T, Cfg::kS><<<dim3((unsigned)wgs), dim3(512), Cfg::kLds, s>>>(
         A, grp.W[0], grp.N[0], grp.kg[0], grp.begin[1], grp.begin[2], grp.begin[3], (int)M, (int)K, grp.C[0],
         grp.ctr[0], ws.part, ws.cnt, grp);
     return hipGetLastError();
