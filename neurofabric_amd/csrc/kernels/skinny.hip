@@ -16,14 +16,17 @@
 // activations through registers) or three smaller ones with the activations
 // through registers (f32) in flight.
 //
+// (f16 batches of 65 to 128 rows: a chunk is 64 KB of activations and 9 KB of
+// Q4_0 codes, so the ring has two stages only and waits for each.)
+//
 // Measured on MI355X against them (us per launch, graph replay over rotated
-// weights; before -> now):
-//   f16 Q4_0  8192x28672  M = 16 / 32 / 64   53.5 / 61.5 / 71.9 -> 34 / 44 / 56
-//   f16 Q8_0  4096x14336  M = 16 / 32 / 64   25.2 / 48.0 / 55.5 -> 17.5 / 20 / 26
-//   f16 Q4_0  4096x4096   M = 16 / 64 / 128  10.3 / 21.1 / 21.9 -> 6.7 / 10.8 / 16.7
-//   f32 Q8_0  14336x4096  M = 16 / 32        23.7 / 31.6 -> 20.4 / 25.9
-//   f32 Q4_0  4096x4096   M = 16 / 64        11.8 / 21.9 -> 9.1 / 15.5
-//   f32 Q4_0  2048x2048   M = 16 / 64         8.0 / 15.8 -> 6.3 / 9.6
+// weights; before -> now; the first line from bench.py, the others one sweep):
+//   f16 Q4_0  8192x28672  M = 16 / 32 / 64   56.4 / 61.8 / 69.7 -> 42.2 / 49.7 / 61.2
+//   f16 Q8_0  4096x14336  M = 16 / 32 / 64   25.6 / 47.1 / 54.9 -> 19.5 / 21.5 / 26.9
+//   f16 Q4_0  4096x4096   M = 16 / 64 / 128  11.3 / 22.3 / 23.5 -> 9.0 / 12.1 / 18.8
+//   f32 Q8_0  14336x4096  M = 16 / 32        24.2 / 34.0 -> 22.3 / 28.3
+//   f32 Q4_0  4096x4096   M = 16             13.0 -> 10.6
+//   f32 Q4_0  2048x2048   M = 16 / 64         9.1 / 16.6 -> 7.5 / 11.0
 //
 // MFMA v_mfma_f32_16x16x32 (f16 or bf16 operands): A = activations (16 rows
 // of M), B = weights (16 rows of N), D[m][n] = sum over 32 k.  Lane l holds
@@ -477,8 +480,9 @@ __global__ __launch_bounds__(64 * kSkWaves) void skinny_kernel(const XT* __restr
 // workgroups; the fix-up of a K split; no less than the bytes at the rate
 // the stream reaches.  The coefficients are least-squares fits to about 700
 // launches per format and type on MI355X (16 shapes from 512 x 1024 to 28672
-// x 8192, 4 to 128 rows, every variant, 1 to 8 K splits); over those the
-// model's pick was within 1-5 % of the fastest on average (worst 1.35 x).
+// x 8192, 4 to 128 rows, every variant, 1 to 8 K splits).  Over the 35 shapes
+// of profiles/skinny_variant_sweep.csv the pick is within 0.2-8 % of the
+// fastest on average (worst 1.30 x: f16 Q8_0 2048x2048 M = 32).
 struct SkCost {
   float chunk, codes, xkb, prod;  // per chunk
   float base, split, round, tbs;  // launch, K split, further rounds; TB/s

@@ -76,30 +76,23 @@ struct LayerParams {
 // each have their own), the tiled MFMA GEMM above (f16: fp16 MFMA; f32:
 // bf16-piece MFMA, K % 64 == 0, else the GEMV).  For f16 the default
 // skinny_max_m is no plain switch point: see skinny_f16_faster() in plan.cpp.
-// Defaults from measured sweeps on MI355X (graph replay over 4 rotated weight
-// copies).  bench.py's configs[4] section (28672x8192 and 8192x28672 Q4_0,
-// f16 activations): the GEMV is fastest up to M = 2 (31.0 / 38.8 us against
-// 46.3 / 47.1 us for the small-batch kernel at 28672x8192) while two of its
-// workgroups fit a CU's LDS (at 8192x28672 M = 2 its 112 KB activation stage
-// leaves one: 47.9 against 46.3 us; plan.cpp), the small-batch kernel for M = 4..16 (58.6 and
-// 61.6 us at M = 16 against 67.6 and 69.2 us for the tiled GEMM), the tiled
-// GEMM from M = 32 (70.2 vs 88.8 us and 69.4 vs 88.7 us).  f32 activations
-// (configs[3] Llama-3-8B Q8_0 step): the small-batch ring kernel up to
-// M = 64, all rows in one launch (5.12 against 11.75 ms per M = 64 step and
-// 4.86 against 11.64 ms at M = 48 with the bf16-piece tiled GEMM), the tiled
-// GEMM above, where the ring kernel does not go.
-// At M = 3..4 the winner depends on the weight size: the GEMV wins on
-// matrices up to about 10 MB, where the small-batch kernel's fixed
-// per-launch cost dominates (f32 M = 4: 2048x2048 4.9 vs 8.6 us, 4096x4096
-// 10.4 vs 11.4 us; f16 5632x2048 6.5 vs 8.7 us), they tie at 25 MB
-// (11008x4096 f32 20.2 vs 18.5, 4096x11008 19.5 vs 19.2 us) and the
-// small-batch kernel wins beyond (32000x2048 f32 25.0 vs 21.4 us,
-// 32000x4096 49.3 vs 36.2 us; f16 alike).  Hence the GEMV takes M = 3..4
-// only while the weights are at most gemv_m4_max_weight_bytes (16 MB).
+// Defaults from measured sweeps on MI355X (graph replay over rotated weight
+// copies; us, GEMV / small-batch).  M = 1: the GEMV everywhere (Q4_0 f16
+// 28672x8192 28.1 / 34.8).  M = 2: the GEMV while two of its workgroups fit a
+// CU's LDS (gemv_m2_max_stage_bytes: Q4_0 f16 14336x4096 11.9 / 13.6,
+// 28672x8192 35.2 / 34.8; past it 8192x28672 42.5 / 40.9, f32 4096x14336 22.0 /
+// 17.3).  M = 3..4: it depends on the weight size, the GEMV's time growing with
+// the rows and the small-batch kernel's not (gemv_m4_max_weight_bytes, 16 MB):
+// at M = 4 Q4_0 f32 2048x2048 5.6 / 7.0, 5632x2048 7.4 / 9.5, 4096x4096 (9.4
+// MB) 10.8 / 10.1, 6144x4096 (14 MB) 13.2 / 11.8, 11008x4096 18.7 / 15.4; f16
+// 4096x4096 7.6 / 8.5, 6144x4096 9.6 / 8.9, 11008x4096 13.9 / 13.1; Q8_0 crosses
+// later, f32 6144x4096 (27 MB) 12.6 / 13.1, 8192x4096 (36 MB) 15.5 / 14.0, f16
+// 11008x4096 (48 MB) 15.8 / 16.3.  f32 activations: the small-batch kernels up
+// to M = 64, all rows in one launch (a Llama-3-8B Q8_0 step at M = 64 5.12
+// against 11.75 ms with the bf16-piece tiled GEMM), the tiled GEMM above.
 // skinny_f16_max_k caps K for f16 batches above M = 4 on the small-batch
-// kernel (longer K goes to the tiled GEMM); no cap by default, since the
-// small-batch kernel's K split over workgroups makes it the
-// faster one at K = 28672 too (M = 8: 52.8 against 68.1 us).
+// kernel (longer K goes to the tiled GEMM); no cap by default: at K = 28672 M
+// = 8 the small-batch kernel takes 41.0 us, the tiled one 60.4.
 constexpr uint32_t kSkinnyMaxMF16 = 128;  // the rows of one launch
 struct Tuning {
   uint32_t gemv_max_m_f32 = 4;
